@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define PARROT_ABI_VERSION 14
+#define PARROT_ABI_VERSION 15
 
 #define PARROT_OK 0
 #define PARROT_ERR_NULL_POINTER (-1)
@@ -238,6 +238,38 @@ int parrot_decode_attention_latent_f32(const float* q, const void* latent_new, v
                                        const int32_t* position, int32_t batch, int32_t heads,
                                        int32_t latent_dim, int32_t max_positions, float scale,
                                        float* out, void* stream);
+
+/* The three decode attentions above with the keys split over workgroups, for
+ * long contexts: the same stores and, up to fp32 summation order, the same
+ * results, in two launches (64 keys of one kv head per workgroup, then a
+ * merge per head).  Additionally head_dim % 32 == 0, heads / kv_heads <= 16,
+ * min(window, max_positions) <= 16384, batch <= 65535, q 16-byte aligned, and
+ * a 16-byte aligned workspace of
+ * parrot_decode_attention_split_workspace_bytes (0 for an unsupported shape;
+ * the latent form's kv_heads is 1, its window max_positions), which holds
+ * nothing between calls.  Every position is valid: the split is sized for
+ * the window and chunks past the position do nothing.  Interfaces replaced:
+ * as the forms above. */
+size_t parrot_decode_attention_split_workspace_bytes(int32_t batch, int32_t heads,
+                                                     int32_t kv_heads, int32_t head_dim,
+                                                     int32_t max_positions, int32_t window);
+int parrot_decode_attention_split_bf16(const void* q, const void* k_new, const void* v_new,
+                                       void* key_cache, void* value_cache,
+                                       const int32_t* position, int32_t batch, int32_t heads,
+                                       int32_t kv_heads, int32_t head_dim, int32_t max_positions,
+                                       int32_t window, float scale, void* out, void* workspace,
+                                       size_t workspace_bytes, void* stream);
+int parrot_decode_attention_heads_split_bf16(
+    const void* q, const void* k_new, const void* v_new, void* key_cache, void* value_cache,
+    const int32_t* position, int32_t batch, int32_t heads, int32_t kv_heads, int32_t head_dim,
+    int32_t max_positions, int32_t window, float scale, const void* out_weight, int32_t dim,
+    float* contributions, void* workspace, size_t workspace_bytes, void* stream);
+int parrot_decode_attention_latent_split_f32(const float* q, const void* latent_new,
+                                             void* latent_cache, const int32_t* position,
+                                             int32_t batch, int32_t heads, int32_t latent_dim,
+                                             int32_t max_positions, float scale, float* out,
+                                             void* workspace, size_t workspace_bytes,
+                                             void* stream);
 
 /* The decode step's q|k|v projection of a local (GQA) layer with RoPE, one
  * launch: for each token t, q|k|v = h_t W^T rounded to bf16 (qkv_weight

@@ -13,6 +13,7 @@ from __future__ import annotations
 import torch
 from torch import Tensor
 
+from . import hip_moe
 from .model import GenerationState, Parrot
 
 
@@ -47,16 +48,34 @@ class DecodeGraph:
         # One eager step on a side stream fills every lazily built cache
         # (packed weights, absorbed maps, RoPE tables, scratch buffers);
         # its cache row at `start` is rewritten by the first real step.
+        # The step's attention splits the keys of long contexts over workgroups
+        # (hip_moe.decode_splits), a choice of launches made when a graph is
+        # captured: one graph per form, the second captured when the position
+        # first needs it.
+        self.out: Tensor | None = None
+        self.graphs: dict[bool, torch.cuda.CUDAGraph] = {}
+        self._capture(start)
+
+    def _splits(self) -> bool:
+        return hip_moe.decode_splits(self.state.position + 1, self.state.batch_size)
+
+    def _capture(self, start: int) -> None:
+        device = self.ids.device
         side = torch.cuda.Stream(device)
         side.wait_stream(torch.cuda.current_stream(device))
         with torch.cuda.stream(side):
             self._run()
         torch.cuda.current_stream(device).wait_stream(side)
         self._rewind(start)
-        self.graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(self.graph):
-            self.out = self._run()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = self._run()
+            if self.out is None:
+                self.out = out
+            elif out.data_ptr() != self.out.data_ptr():
+                self.out.copy_(out)  # every graph's output is the same tensor
         self._rewind(start)
+        self.graphs[self._splits()] = graph
 
     def _run(self) -> Tensor:
         if self.logits:
@@ -78,8 +97,12 @@ class DecodeGraph:
             raise ValueError("decode input must be [cached batch, 1]")
         if self.state.position >= self.model.config.max_seq_len:
             raise ValueError("Generation state has reached max_seq_len")
+        splits = self._splits()
+        if splits not in self.graphs:
+            input_ids = input_ids.clone()  # the eager step may write self.ids
+            self._capture(self.state.position)
         if input_ids.data_ptr() != self.ids.data_ptr():
             self.ids.copy_(input_ids)
-        self.graph.replay()
+        self.graphs[splits].replay()
         self.state.position += 1
         return self.out

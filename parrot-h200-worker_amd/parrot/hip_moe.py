@@ -957,12 +957,44 @@ def _check_position(position: Tensor, device: torch.device) -> None:
         raise RuntimeError("position must be a one-element int32 tensor on the cache's device")
 
 
+def decode_splits(context: int | None, batch: int, window: int | None = None) -> bool:
+    """Whether decode attention over ``context`` positions (the new one
+    included; None: unknown) splits its keys over workgroups and merges (two
+    launches) instead of streaming them through one workgroup per head.  Both
+    forms are right at every position: the choice is one of speed.
+
+    The split form's time hardly depends on the context, but grows with the
+    batch (its launch covers the whole window), so the line does too.
+    Measured on MI355X in graphs (8 heads; one launch / split, us):
+    local layers b = 1 256 keys 6.7 / 7.9, 384 9.2 / 7.9, 2048 28.4 / 8.2;
+    b = 8 384 7.9 / 8.2, 512 8.9 / 8.4, 2048 31.5 / 9.4; latent layers b = 4
+    320 8.8 / 8.9, 512 11.1 / 8.8, 3900 63.6 / 9.7; b = 12 512 11.1 / 12.9,
+    1024 19.6 / 13.1, 3900 74.5 / 15.7."""
+    if context is None:
+        return False
+    return (context if window is None else min(context, window)) > 320 + 32 * min(batch, 22)
+
+
+def _split_workspace(q: Tensor, batch: int, heads: int, kv_heads: int, head_dim: int,
+                     max_pos: int, window: int, context: int | None) -> Tensor | None:
+    """The split form's workspace (a fresh one per call: calls on several
+    streams share nothing), or None where the one-launch form runs."""
+    if not decode_splits(context, batch, window) or q.data_ptr() % 16:
+        return None
+    nbytes = _abi.load().parrot_decode_attention_split_workspace_bytes(
+        batch, heads, kv_heads, head_dim, max_pos, window)
+    if nbytes == 0:
+        return None
+    return torch.empty(nbytes, dtype=torch.uint8, device=q.device)
+
+
 def decode_attention(q: Tensor, k_new: Tensor, v_new: Tensor, key_cache: Tensor,
                      value_cache: Tensor, position: Tensor, window: int,
-                     scale: float) -> Tensor:
+                     scale: float, context: int | None = None) -> Tensor:
     """One decode step of sliding-window GQA: store k_new / v_new [b, Hk, 1, d]
     at cache position p = position (device int32) and attend q [b, H, 1, d]
-    over positions max(0, p - window + 1) .. p.  Returns [b, H * d] bf16."""
+    over positions max(0, p - window + 1) .. p.  Returns [b, H * d] bf16.
+    ``context``: p + 1 where the host knows it (see ``decode_splits``)."""
     _require(q, "HIP decode attention")
     b, heads, t, d = q.shape
     _, kv_heads, max_pos, _ = key_cache.shape
@@ -975,10 +1007,15 @@ def decode_attention(q: Tensor, k_new: Tensor, v_new: Tensor, key_cache: Tensor,
     _check_position(position, q.device)
     q, k_new, v_new = q.contiguous(), k_new.contiguous(), v_new.contiguous()
     out = q.new_empty((b, heads * d))
-    _abi.check(_abi.load().parrot_decode_attention_bf16(
-        ptr(q), ptr(k_new), ptr(v_new), ptr(key_cache), ptr(value_cache), ptr(position),
-        b, heads, kv_heads, d, max_pos, window, scale, ptr(out), _stream(q.device)),
-        "parrot_decode_attention_bf16")
+    args = (ptr(q), ptr(k_new), ptr(v_new), ptr(key_cache), ptr(value_cache), ptr(position),
+            b, heads, kv_heads, d, max_pos, window, scale, ptr(out))
+    ws = _split_workspace(q, b, heads, kv_heads, d, max_pos, window, context)
+    if ws is not None:
+        _abi.check(_abi.load().parrot_decode_attention_split_bf16(
+            *args, ptr(ws), ws.numel(), _stream(q.device)), "parrot_decode_attention_split_bf16")
+        return out
+    _abi.check(_abi.load().parrot_decode_attention_bf16(*args, _stream(q.device)),
+               "parrot_decode_attention_bf16")
     return out
 
 
@@ -1003,7 +1040,7 @@ def decode_attention_heads_supported(tokens: int, dim: int, heads: int, kv_heads
 
 def decode_attention_heads(q: Tensor, k_new: Tensor, v_new: Tensor, key_cache: Tensor,
                            value_cache: Tensor, position: Tensor, window: int, scale: float,
-                           out_weight: Tensor) -> Tensor:
+                           out_weight: Tensor, context: int | None = None) -> Tensor:
     """``decode_attention`` with the output projection deferred per head (the
     reference's defer_sum, parrot/model.py:301-316): returns contributions
     [b, H, dim] fp32, contributions[b, h] = y_bf16[b, h] @ out_weight[:, h d :
@@ -1027,10 +1064,16 @@ def decode_attention_heads(q: Tensor, k_new: Tensor, v_new: Tensor, key_cache: T
     _check_position(position, q.device)
     q, k_new, v_new = q.contiguous(), k_new.contiguous(), v_new.contiguous()
     out = torch.empty((b, heads, dim), dtype=torch.float32, device=q.device)
-    _abi.check(_abi.load().parrot_decode_attention_heads_bf16(
-        ptr(q), ptr(k_new), ptr(v_new), ptr(key_cache), ptr(value_cache), ptr(position),
-        b, heads, kv_heads, d, max_pos, window, scale, ptr(out_weight), dim, ptr(out),
-        _stream(q.device)), "parrot_decode_attention_heads_bf16")
+    args = (ptr(q), ptr(k_new), ptr(v_new), ptr(key_cache), ptr(value_cache), ptr(position),
+            b, heads, kv_heads, d, max_pos, window, scale, ptr(out_weight), dim, ptr(out))
+    ws = _split_workspace(q, b, heads, kv_heads, d, max_pos, window, context)
+    if ws is not None:
+        _abi.check(_abi.load().parrot_decode_attention_heads_split_bf16(
+            *args, ptr(ws), ws.numel(), _stream(q.device)),
+            "parrot_decode_attention_heads_split_bf16")
+        return out
+    _abi.check(_abi.load().parrot_decode_attention_heads_bf16(*args, _stream(q.device)),
+               "parrot_decode_attention_heads_bf16")
     return out
 
 
@@ -1228,7 +1271,8 @@ def mla_decode_out(context: Tensor, absorbed_output: Tensor,
 
 
 def decode_attention_latent(q: Tensor, latent_new: Tensor, latent_cache: Tensor,
-                            position: Tensor, heads: int, scale: float) -> Tensor:
+                            position: Tensor, heads: int, scale: float,
+                            context: int | None = None) -> Tensor:
     """One MLA decode step over the latent cache: store latent_new [b, 1, r]
     at position p and attend the fp32 absorbed queries q [b, 1, H * r] over
     latents 0 .. p (keys = values).  Returns the fp32 context [b, H * r]."""
@@ -1243,9 +1287,16 @@ def decode_attention_latent(q: Tensor, latent_new: Tensor, latent_cache: Tensor,
     _check_position(position, q.device)
     q, latent_new = q.contiguous(), latent_new.contiguous()
     out = q.new_empty((b, heads * r))
-    _abi.check(_abi.load().parrot_decode_attention_latent_f32(
-        ptr(q), ptr(latent_new), ptr(latent_cache), ptr(position), b, heads, r, max_pos, scale,
-        ptr(out), _stream(q.device)), "parrot_decode_attention_latent_f32")
+    args = (ptr(q), ptr(latent_new), ptr(latent_cache), ptr(position), b, heads, r, max_pos,
+            scale, ptr(out))
+    ws = _split_workspace(q, b, heads, 1, r, max_pos, max_pos, context)
+    if ws is not None:
+        _abi.check(_abi.load().parrot_decode_attention_latent_split_f32(
+            *args, ptr(ws), ws.numel(), _stream(q.device)),
+            "parrot_decode_attention_latent_split_f32")
+        return out
+    _abi.check(_abi.load().parrot_decode_attention_latent_f32(*args, _stream(q.device)),
+               "parrot_decode_attention_latent_f32")
     return out
 
 

@@ -342,6 +342,94 @@ int parrot_decode_attention_latent_f32(const float* q, const void* latent_new, v
       position, batch, heads, latent_dim, max_positions, scale, out, as_stream(stream)));
 }
 
+static int check_decode_split(int32_t heads, int32_t kv_heads, int32_t head_dim,
+                              int32_t max_positions, int32_t window, int32_t batch,
+                              const void* q, const void* workspace, size_t workspace_bytes) {
+  if (!parrot::decode_split_supported(heads, kv_heads, head_dim, max_positions, window))
+    return PARROT_ERR_UNSUPPORTED;
+  if (batch > 65535) return PARROT_ERR_UNSUPPORTED;
+  if (!workspace || workspace_bytes < parrot::decode_split_workspace_bytes(
+                                          batch, heads, head_dim, max_positions, window))
+    return PARROT_ERR_WORKSPACE;
+  if (!aligned16(q) || !aligned16(workspace)) return PARROT_ERR_ALIGNMENT;
+  return PARROT_OK;
+}
+
+size_t parrot_decode_attention_split_workspace_bytes(int32_t batch, int32_t heads,
+                                                     int32_t kv_heads, int32_t head_dim,
+                                                     int32_t max_positions, int32_t window) {
+  if (check_decode_shape(batch, heads, kv_heads, head_dim, max_positions, window) != PARROT_OK ||
+      !parrot::decode_split_supported(heads, kv_heads, head_dim, max_positions, window))
+    return 0;
+  return parrot::decode_split_workspace_bytes(batch, heads, head_dim, max_positions, window);
+}
+
+int parrot_decode_attention_split_bf16(const void* q, const void* k_new, const void* v_new,
+                                       void* key_cache, void* value_cache,
+                                       const int32_t* position, int32_t batch, int32_t heads,
+                                       int32_t kv_heads, int32_t head_dim, int32_t max_positions,
+                                       int32_t window, float scale, void* out, void* workspace,
+                                       size_t workspace_bytes, void* stream) {
+  if (!q || !k_new || !v_new || !key_cache || !value_cache || !position || !out)
+    return PARROT_ERR_NULL_POINTER;
+  if (int rc = check_decode_shape(batch, heads, kv_heads, head_dim, max_positions, window))
+    return rc;
+  if (!aligned16(k_new) || !aligned16(v_new) || !aligned16(key_cache) || !aligned16(value_cache))
+    return PARROT_ERR_ALIGNMENT;
+  if (int rc = check_decode_split(heads, kv_heads, head_dim, max_positions, window, batch, q,
+                                  workspace, workspace_bytes))
+    return rc;
+  return status(parrot::launch_decode_attention_split(
+      static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k_new),
+      static_cast<const uint16_t*>(v_new), static_cast<uint16_t*>(key_cache),
+      static_cast<uint16_t*>(value_cache), position, batch, heads, kv_heads, head_dim,
+      max_positions, window, scale, static_cast<uint16_t*>(out), workspace, as_stream(stream)));
+}
+
+int parrot_decode_attention_heads_split_bf16(
+    const void* q, const void* k_new, const void* v_new, void* key_cache, void* value_cache,
+    const int32_t* position, int32_t batch, int32_t heads, int32_t kv_heads, int32_t head_dim,
+    int32_t max_positions, int32_t window, float scale, const void* out_weight, int32_t dim,
+    float* contributions, void* workspace, size_t workspace_bytes, void* stream) {
+  if (!q || !k_new || !v_new || !key_cache || !value_cache || !position || !out_weight ||
+      !contributions)
+    return PARROT_ERR_NULL_POINTER;
+  if (int rc = check_decode_heads_shape(batch, heads, kv_heads, head_dim, max_positions, window,
+                                        dim))
+    return rc;
+  if (!aligned16(k_new) || !aligned16(v_new) || !aligned16(key_cache) ||
+      !aligned16(value_cache) || !aligned16(out_weight))
+    return PARROT_ERR_ALIGNMENT;
+  if (int rc = check_decode_split(heads, kv_heads, head_dim, max_positions, window, batch, q,
+                                  workspace, workspace_bytes))
+    return rc;
+  return status(parrot::launch_decode_attention_heads_split(
+      static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k_new),
+      static_cast<const uint16_t*>(v_new), static_cast<uint16_t*>(key_cache),
+      static_cast<uint16_t*>(value_cache), position, batch, heads, kv_heads, head_dim,
+      max_positions, window, scale, static_cast<const uint16_t*>(out_weight), dim, contributions,
+      workspace, as_stream(stream)));
+}
+
+int parrot_decode_attention_latent_split_f32(const float* q, const void* latent_new,
+                                             void* latent_cache, const int32_t* position,
+                                             int32_t batch, int32_t heads, int32_t latent_dim,
+                                             int32_t max_positions, float scale, float* out,
+                                             void* workspace, size_t workspace_bytes,
+                                             void* stream) {
+  if (!q || !latent_new || !latent_cache || !position || !out) return PARROT_ERR_NULL_POINTER;
+  if (int rc = check_decode_shape(batch, heads, 1, latent_dim, max_positions, max_positions))
+    return rc;
+  if (!aligned16(latent_new) || !aligned16(latent_cache)) return PARROT_ERR_ALIGNMENT;
+  if (int rc = check_decode_split(heads, 1, latent_dim, max_positions, max_positions, batch, q,
+                                  workspace, workspace_bytes))
+    return rc;
+  return status(parrot::launch_decode_attention_latent_split(
+      q, static_cast<const uint16_t*>(latent_new), static_cast<uint16_t*>(latent_cache),
+      position, batch, heads, latent_dim, max_positions, scale, out, workspace,
+      as_stream(stream)));
+}
+
 // The depth mix a decode launch makes its input rows with: checks and fills
 // `mix` from the sources (as parrot_depth_mix_bf16 takes them) and the norms.
 static int make_decode_mix(const void* const* sources, int32_t n_sources, const void* query,

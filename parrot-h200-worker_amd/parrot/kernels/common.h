@@ -452,6 +452,28 @@ hipError_t launch_decode_attention_heads(const uint16_t* q, const uint16_t* k_ne
                                          int heads, int kv_heads, int head_dim, int max_pos,
                                          int window, float scale, const uint16_t* out_weight,
                                          int dim, float* contributions, hipStream_t s);
+// The same three with the keys split over workgroups and merged by a second
+// launch, for long contexts; head_dim a multiple of 32 and at most 16 query
+// heads per kv head.  q 16-byte aligned; workspace 16-byte aligned, of
+// decode_split_workspace_bytes.
+bool decode_split_supported(int heads, int kv_heads, int head_dim, int max_pos, int window);
+size_t decode_split_workspace_bytes(int batch, int heads, int head_dim, int max_pos, int window);
+hipError_t launch_decode_attention_split(const uint16_t* q, const uint16_t* k_new,
+                                         const uint16_t* v_new, uint16_t* k_cache,
+                                         uint16_t* v_cache, const int32_t* position, int batch,
+                                         int heads, int kv_heads, int head_dim, int max_pos,
+                                         int window, float scale, uint16_t* out,
+                                         void* workspace, hipStream_t s);
+hipError_t launch_decode_attention_heads_split(
+    const uint16_t* q, const uint16_t* k_new, const uint16_t* v_new, uint16_t* k_cache,
+    uint16_t* v_cache, const int32_t* position, int batch, int heads, int kv_heads, int head_dim,
+    int max_pos, int window, float scale, const uint16_t* out_weight, int dim,
+    float* contributions, void* workspace, hipStream_t s);
+hipError_t launch_decode_attention_latent_split(const float* q, const uint16_t* latent_new,
+                                                uint16_t* latent_cache, const int32_t* position,
+                                                int batch, int heads, int latent_dim,
+                                                int max_pos, float scale, float* out,
+                                                void* workspace, hipStream_t s);
 size_t mla_decode_lds_bytes(int tokens, int k, int elem_bytes);
 hipError_t launch_decode_linear(const uint16_t* x, int tokens, int k, const uint16_t* w, int n,
                                 const uint16_t* addend, uint16_t* out, hipStream_t s);

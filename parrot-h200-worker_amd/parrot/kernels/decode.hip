@@ -310,6 +310,351 @@ hipError_t launch_decode(const QT* q, const uint16_t* k_new, const uint16_t* v_n
   return hipGetLastError();
 }
 
+// ---------------------------------------------------------------------------
+// Long contexts: the keys split over workgroups.
+//
+// One workgroup per (head, sequence) streams the whole window through one
+// CU: 28.8 us at 2048 keys (b = 1), 31.6 us (b = 8) and 65 us for the latent
+// layers at 3900 keys (b = 4), for 0.8-4 MB that the chip reads in 1-2 us.
+// Here a workgroup takes kSplitKeys = 64 consecutive keys of one kv head for
+// all the query heads that share it, so each row is read once (not once per
+// head), and leaves (max, sum, unnormalised output) per head in a workspace;
+// a second launch merges a head's chunks in chunk order and, for the deferred
+// residual, projects its share of the output columns as the one-launch kernel
+// does.  64 keys give b = 1 64 workgroups at the 2048-key window and b = 8
+// 512; the launch is sized for the whole window, chunks past the position
+// exit at once.
+//
+//   scores    v_mfma_f32_16x16x32_bf16, A = the group's query heads (rows
+//             past them zero), B = 16 keys per wavefront straight from the
+//             cache rows.  An fp32 query (latent layers) enters as three bf16
+//             parts that add up to it exactly, accumulated in fp32, so the
+//             products are as exact as the fp32 dot's.
+//   softmax   one key per lane per head, fp32, within the wavefront that owns
+//             the head.
+//   values    staged in LDS once; wavefront w sums heads w, w + 4, ... in
+//             fp32 over (key slot, 16-byte chunk) lanes.
+constexpr int kSplitKeys = 64;
+constexpr int kSplitMaxChunks = 256;  // chunk weights the merge keeps in LDS
+
+// A 16-byte fragment (8 values) of a query row as bf16 parts whose sum is the
+// row: one part for a bf16 query, three for an fp32 one (8 + 8 + 8 bits).
+template <typename QT>
+constexpr int kQueryParts = sizeof(QT) == 4 ? 3 : 1;
+
+__device__ __forceinline__ void query_parts(const uint16_t* p, bool live, bf16x8 (&part)[1]) {
+  const uint4 v = *reinterpret_cast<const uint4*>(p);
+  part[0] = __builtin_bit_cast(bf16x8, live ? v : make_uint4(0u, 0u, 0u, 0u));
+}
+
+__device__ __forceinline__ void query_parts(const float* p, bool live, bf16x8 (&part)[3]) {
+  const float4 a = reinterpret_cast<const float4*>(p)[0];
+  const float4 b = reinterpret_cast<const float4*>(p)[1];
+  const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+  uint32_t w[3][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+#pragma unroll
+    for (int t = 0; t < 3; ++t) w[t][i] = 0u;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      float rest = live ? v[2 * i + j] : 0.0f;
+#pragma unroll
+      for (int t = 0; t < 3; ++t) {
+        const uint16_t h = f32_to_bf16(rest);
+        w[t][i] |= static_cast<uint32_t>(h) << (16 * j);
+        // An infinite part leaves no remainder (inf - inf would be NaN).
+        const float part_v = bf16_to_f32(h);
+        rest = __builtin_isinf(part_v) ? 0.0f : rest - part_v;
+      }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < 3; ++t)
+    part[t] = __builtin_bit_cast(bf16x8, make_uint4(w[t][0], w[t][1], w[t][2], w[t][3]));
+}
+
+// CH = head_dim / 8 (a multiple of 4); HPW = query heads per wavefront,
+// heads / kv_heads <= 4 HPW <= 16.
+template <typename QT, int CH, int HPW>
+__global__ __launch_bounds__(256) void decode_split_kernel(
+    const QT* __restrict__ q, const uint16_t* __restrict__ k_new,
+    const uint16_t* __restrict__ v_new, uint16_t* __restrict__ k_cache,
+    uint16_t* __restrict__ v_cache, const int32_t* __restrict__ position, int heads,
+    int kv_heads, int max_pos, int window, float scale, float2* __restrict__ part_ml,
+    float* __restrict__ part_o) {
+  constexpr int D = CH * 8;
+  constexpr int KS = D / 32;             // MFMA k steps of a score
+  constexpr int kLanes = CH <= 16 ? 16 : 32;  // lanes per key slot in the value pass
+  constexpr int kSlots = kWave / kLanes;      // key slots per wavefront
+  constexpr int kParts = kQueryParts<QT>;
+  constexpr int kPieces = kSplitKeys * CH / 256;  // value pieces staged per thread
+  __shared__ __attribute__((aligned(16))) uint16_t v_s[kSplitKeys * D];
+  __shared__ float s_s[4 * HPW][kSplitKeys];
+
+  asm volatile("" ::"s"(q), "s"(k_new), "s"(v_new), "s"(k_cache), "s"(v_cache), "s"(position),
+               "s"(heads), "s"(kv_heads), "s"(max_pos), "s"(window), "s"(scale), "s"(part_ml),
+               "s"(part_o));
+  using const_i32 = const __attribute__((address_space(4))) int32_t;
+  const int pos = *(const_i32*)(reinterpret_cast<uintptr_t>(position));
+  const int chunk = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
+  if (pos < 0 || pos >= max_pos) return;  // uniform: nothing to attend to
+  const int lo = max(0, pos - window + 1);
+  const int L = pos - lo + 1;
+  const int c0 = chunk * kSplitKeys;
+  if (c0 >= L) return;  // uniform: no keys here
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rep = heads / kv_heads;
+
+  const int64_t kv_index = static_cast<int64_t>(b) * kv_heads + kvh;
+  const uint16_t* kn = k_new + kv_index * D;
+  const uint16_t* vn = v_new + kv_index * D;
+  uint16_t* kc = k_cache + kv_index * max_pos * D;
+  uint16_t* vc = v_cache + kv_index * max_pos * D;
+  // Keys past the last one (of the final chunk) read its row; their scores
+  // are masked below.  The row at `pos` comes from the new rows.
+  auto row = [&](const uint16_t* cache, const uint16_t* fresh, int j) -> const uint16_t* {
+    const int key = lo + min(j, L - 1);
+    return key == pos ? fresh : cache + static_cast<int64_t>(key) * D;
+  };
+
+  // Every load first: this wavefront's 16 keys, the query heads, the values.
+  const int g = lane >> 4, c = lane & 15;
+  bf16x8 kf[KS];
+  {
+    const uint16_t* kr = row(kc, kn, c0 + 16 * wave + c) + 8 * g;
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+      kf[s] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(kr + 32 * s));
+  }
+  const QT* qrow = q + (static_cast<int64_t>(b) * heads + kvh * rep + min(c, rep - 1)) * D + 8 * g;
+  uint4 vr[kPieces];
+#pragma unroll
+  for (int i = 0; i < kPieces; ++i) {
+    const int piece = i * 256 + tid;
+    vr[i] = *reinterpret_cast<const uint4*>(row(vc, vn, c0 + piece / CH) + (piece % CH) * 8);
+  }
+  f32x4 sc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    bf16x8 part[kParts];
+    query_parts(qrow + 32 * s, c < rep, part);
+#pragma unroll
+    for (int t = kParts - 1; t >= 0; --t)  // small parts first
+      sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(part[t], kf[s], sc, 0, 0, 0);
+  }
+  // The chunk that holds `pos` stores the new rows.
+  if (c0 + kSplitKeys >= L && tid < D) {
+    kc[static_cast<int64_t>(pos) * D + tid] = kn[tid];
+    if (v_cache != k_cache) vc[static_cast<int64_t>(pos) * D + tid] = vn[tid];
+  }
+#pragma unroll
+  for (int i = 0; i < kPieces; ++i)
+    *reinterpret_cast<uint4*>(v_s + (i * 256 + tid) * 8) = vr[i];
+  // C fragment: lane holds key c of the wavefront's 16, heads 4 g + r.
+  const bool valid = c0 + 16 * wave + c < L;
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (4 * g + r < 4 * HPW) s_s[4 * g + r][16 * wave + c] = valid ? sc[r] * scale : -INFINITY;
+  __syncthreads();
+
+  const int64_t part0 = (static_cast<int64_t>(b) * heads + kvh * rep) * gridDim.x + chunk;
+  const int slot = lane / kLanes, vch = lane % kLanes;
+  float acc[HPW][8];
+#pragma unroll
+  for (int i = 0; i < HPW; ++i) {
+    const int h = wave + 4 * i;
+    const float v = s_s[h][lane];
+    const float m = wave_max(v);
+    // A chunk whose scores are all -inf weighs nothing.
+    const float e = m == -INFINITY ? 0.0f : __expf(v - m);
+    const float l = wave_sum(e);
+    s_s[h][lane] = e;  // read back by this wavefront only
+    if (lane == 0 && h < rep)
+      part_ml[part0 + static_cast<int64_t>(h) * gridDim.x] = make_float2(m, l);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) acc[i][k] = 0.0f;
+  }
+  const int vlane = min(vch, CH - 1);
+#pragma unroll 4
+  for (int j = slot; j < kSplitKeys; j += kSlots) {
+    const uint4 x = *reinterpret_cast<const uint4*>(v_s + j * D + vlane * 8);
+    const float xv[8] = {lo_bf16(x.x), hi_bf16(x.x), lo_bf16(x.y), hi_bf16(x.y),
+                         lo_bf16(x.z), hi_bf16(x.z), lo_bf16(x.w), hi_bf16(x.w)};
+#pragma unroll
+    for (int i = 0; i < HPW; ++i) {
+      const float p = s_s[wave + 4 * i][j];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) acc[i][k] += p * xv[k];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < HPW; ++i) {
+    const int h = wave + 4 * i;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      if constexpr (kSlots == 4) acc[i][k] += __shfl_xor(acc[i][k], 16);
+      acc[i][k] += __shfl_xor(acc[i][k], 32);
+    }
+    if (slot == 0 && vch < CH && h < rep) {
+      float4* o = reinterpret_cast<float4*>(
+          part_o + (part0 + static_cast<int64_t>(h) * gridDim.x) * D + vch * 8);
+      o[0] = make_float4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]);
+      o[1] = make_float4(acc[i][4], acc[i][5], acc[i][6], acc[i][7]);
+    }
+  }
+}
+
+// Merges a head's chunks: output = sum_c e^(m_c - M) o_c / sum_c e^(m_c - M)
+// l_c with M = max_c m_c.  Q as in decode_attention_kernel.
+template <typename OT, int CH, int Q>
+__global__ __launch_bounds__(256) void decode_merge_kernel(
+    const float2* __restrict__ part_ml, const float* __restrict__ part_o,
+    const int32_t* __restrict__ position, int heads, int max_pos, int window, int chunks,
+    OT* __restrict__ out, HeadsOut ho) {
+  constexpr int D = CH * 8;
+  constexpr int kVec = D / 4;            // float4 pieces of an output row
+  constexpr int kGroups = 256 / kVec;    // chunks summed side by side
+  constexpr int kPre = 8;                // pieces per thread loaded at entry
+  __shared__ float w_s[kSplitMaxChunks];
+  __shared__ float4 part_s[kGroups][kVec];
+  __shared__ float ob[D];
+  asm volatile("" ::"s"(part_ml), "s"(part_o), "s"(position), "s"(heads), "s"(max_pos),
+               "s"(window), "s"(chunks), "s"(out));
+  if constexpr (Q > 0) asm volatile("" ::"s"(ho.weight), "s"(ho.dim), "s"(ho.contributions));
+  using const_i32 = const __attribute__((address_space(4))) int32_t;
+  const int pos = *(const_i32*)(reinterpret_cast<uintptr_t>(position));
+  const int h = Q > 0 ? static_cast<int>(blockIdx.x) / Q : static_cast<int>(blockIdx.x);
+  const int part_n = Q > 0 ? static_cast<int>(blockIdx.x) % Q : 0;
+  const int b = blockIdx.y;
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int nq = Q > 0 ? ho.dim / Q : 0;
+  if (pos < 0 || pos >= max_pos) return;
+  const int L = min(pos + 1, window);
+  const int n = (L + kSplitKeys - 1) / kSplitKeys;  // live chunks
+  const int64_t row = static_cast<int64_t>(b) * heads + h;
+  const float2* ml = part_ml + row * chunks;
+  const float4* po = reinterpret_cast<const float4*>(part_o + row * chunks * D);
+
+  const float2 ml0 = ml[min(lane, n - 1)];
+  const int vec = tid % kVec, grp = tid / kVec;
+  float4 pre[kPre];
+#pragma unroll
+  for (int u = 0; u < kPre; ++u) pre[u] = po[static_cast<int64_t>(min(grp + u * kGroups, n - 1)) * kVec + vec];
+  uint4 wo[Q > 0 ? CH : 1];
+  if constexpr (Q > 0) {
+    asm volatile("" ::: "memory");
+    const uint4* wrow = reinterpret_cast<const uint4*>(
+        ho.weight + static_cast<int64_t>(part_n * nq + min(tid, nq - 1)) * heads * D + h * D);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) wo[c] = wrow[c];
+  }
+  // Every wavefront derives the same maximum and denominator.
+  float mx = lane < n ? ml0.x : -INFINITY;
+  for (int c = lane + kWave; c < n; c += kWave) mx = fmaxf(mx, ml[c].x);
+  mx = wave_max(mx);
+  float w0 = lane < n ? __expf(ml0.x - mx) : 0.0f;
+  float sum = w0 * (lane < n ? ml0.y : 0.0f);
+  if (tid < n && tid < kWave) w_s[tid] = w0;
+  for (int c = lane + kWave; c < n; c += kWave) {
+    const float2 v = ml[c];
+    const float w = __expf(v.x - mx);
+    if (tid < kWave) w_s[c] = w;
+    sum += w * v.y;
+  }
+  sum = wave_sum(sum);
+  __syncthreads();
+  float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto add = [&](const float4& o, float w) {
+    a.x += w * o.x;
+    a.y += w * o.y;
+    a.z += w * o.z;
+    a.w += w * o.w;
+  };
+  if (grp < kGroups) {
+#pragma unroll
+    for (int u = 0; u < kPre; ++u) {
+      const int c = grp + u * kGroups;
+      if (c < n) add(pre[u], w_s[c]);
+    }
+    for (int c = grp + kPre * kGroups; c < n; c += kGroups) add(po[static_cast<int64_t>(c) * kVec + vec], w_s[c]);
+    part_s[grp][vec] = a;
+  }
+  __syncthreads();
+  const float inv = 1.0f / sum;
+  const float* ps = reinterpret_cast<const float*>(part_s);
+  for (int i = tid; i < D; i += 256) {
+    float o = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kGroups; ++k) o += ps[k * D + i];
+    if constexpr (Q == 0) store_out(out + row * D + i, o * inv);
+    else ob[i] = to_f32(f32_to_bf16(o * inv));
+  }
+  if constexpr (Q > 0) {
+    __syncthreads();
+    if (tid < nq) {
+      float acc = 0.0f;
+#pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        const float* oc = ob + c * 8;
+        acc += lo_bf16(wo[c].x) * oc[0] + hi_bf16(wo[c].x) * oc[1] + lo_bf16(wo[c].y) * oc[2] +
+               hi_bf16(wo[c].y) * oc[3] + lo_bf16(wo[c].z) * oc[4] + hi_bf16(wo[c].z) * oc[5] +
+               lo_bf16(wo[c].w) * oc[6] + hi_bf16(wo[c].w) * oc[7];
+      }
+      ho.contributions[row * ho.dim + part_n * nq + tid] = acc;
+    }
+  }
+}
+
+// (max, sum) entries of the workspace, padded to whole 16-byte pairs so the
+// partial outputs behind them stay aligned.
+size_t decode_split_ml_entries(int batch, int heads, int chunks) {
+  return (static_cast<size_t>(batch) * heads * chunks + 1) / 2 * 2;
+}
+
+int split_chunks(int max_pos, int window) {
+  return ((window < max_pos ? window : max_pos) + kSplitKeys - 1) / kSplitKeys;
+}
+
+template <typename QT, typename OT, int Q>
+hipError_t launch_decode_split(const QT* q, const uint16_t* k_new, const uint16_t* v_new,
+                               uint16_t* k_cache, uint16_t* v_cache, const int32_t* position,
+                               int batch, int heads, int kv_heads, int head_dim, int max_pos,
+                               int window, float scale, OT* out, HeadsOut ho, void* workspace,
+                               hipStream_t s) {
+  const int chunks = split_chunks(max_pos, window);
+  float2* ml = static_cast<float2*>(workspace);
+  float* po = reinterpret_cast<float*>(ml + decode_split_ml_entries(batch, heads, chunks));
+  const dim3 grid(chunks, kv_heads, batch);
+  const dim3 merge_grid(heads * (Q > 0 ? Q : 1), batch);
+  const int rep = heads / kv_heads;
+#define PARROT_SPLIT(CH, HPW)                                                              \
+  decode_split_kernel<QT, CH, HPW><<<grid, 256, 0, s>>>(q, k_new, v_new, k_cache, v_cache, \
+                                                        position, heads, kv_heads, max_pos, \
+                                                        window, scale, ml, po)
+#define PARROT_SPLIT_CH(CH)                                                                \
+  if (rep <= 4) PARROT_SPLIT(CH, 1);                                                       \
+  else if (rep <= 8) PARROT_SPLIT(CH, 2);                                                  \
+  else PARROT_SPLIT(CH, 4);                                                                \
+  decode_merge_kernel<OT, CH, Q><<<merge_grid, 256, 0, s>>>(ml, po, position, heads,       \
+                                                            max_pos, window, chunks, out, ho)
+  switch (head_dim) {
+    case 32: PARROT_SPLIT_CH(4); break;
+    case 64: PARROT_SPLIT_CH(8); break;
+    case 96: PARROT_SPLIT_CH(12); break;
+    case 128: PARROT_SPLIT_CH(16); break;
+    case 192: PARROT_SPLIT_CH(24); break;
+    case 256: PARROT_SPLIT_CH(32); break;
+    default: return hipErrorInvalidValue;
+  }
+#undef PARROT_SPLIT_CH
+#undef PARROT_SPLIT
+  return hipGetLastError();
+}
+
 }  // namespace
 
 bool decode_head_dim_supported(int head_dim) {
@@ -357,6 +702,55 @@ hipError_t launch_decode_attention_latent(const float* q, const uint16_t* latent
   if (batch == 0) return hipSuccess;
   return launch_decode(q, latent_new, latent_new, latent_cache, latent_cache, position, batch,
                        heads, 1, latent_dim, max_pos, max_pos, scale, out, s);
+}
+
+bool decode_split_supported(int heads, int kv_heads, int head_dim, int max_pos, int window) {
+  return head_dim % 32 == 0 && decode_head_dim_supported(head_dim) && heads / kv_heads <= 16 &&
+         split_chunks(max_pos, window) <= kSplitMaxChunks;
+}
+
+size_t decode_split_workspace_bytes(int batch, int heads, int head_dim, int max_pos, int window) {
+  const int chunks = split_chunks(max_pos, window);
+  return decode_split_ml_entries(batch, heads, chunks) * sizeof(float2) +
+         static_cast<size_t>(batch) * heads * chunks * head_dim * sizeof(float);
+}
+
+hipError_t launch_decode_attention_split(const uint16_t* q, const uint16_t* k_new,
+                                         const uint16_t* v_new, uint16_t* k_cache,
+                                         uint16_t* v_cache, const int32_t* position, int batch,
+                                         int heads, int kv_heads, int head_dim, int max_pos,
+                                         int window, float scale, uint16_t* out,
+                                         void* workspace, hipStream_t s) {
+  if (batch == 0) return hipSuccess;
+  return launch_decode_split<uint16_t, uint16_t, 0>(q, k_new, v_new, k_cache, v_cache, position,
+                                                    batch, heads, kv_heads, head_dim, max_pos,
+                                                    window, scale, out, HeadsOut{}, workspace, s);
+}
+
+hipError_t launch_decode_attention_heads_split(
+    const uint16_t* q, const uint16_t* k_new, const uint16_t* v_new, uint16_t* k_cache,
+    uint16_t* v_cache, const int32_t* position, int batch, int heads, int kv_heads, int head_dim,
+    int max_pos, int window, float scale, const uint16_t* out_weight, int dim,
+    float* contributions, void* workspace, hipStream_t s) {
+  if (batch == 0) return hipSuccess;
+  if (dim % kDecodeHeadsParts != 0 || dim / kDecodeHeadsParts > 256)
+    return hipErrorInvalidValue;
+  return launch_decode_split<uint16_t, uint16_t, kDecodeHeadsParts>(
+      q, k_new, v_new, k_cache, v_cache, position, batch, heads, kv_heads, head_dim, max_pos,
+      window, scale, static_cast<uint16_t*>(nullptr), HeadsOut{out_weight, dim, contributions},
+      workspace, s);
+}
+
+hipError_t launch_decode_attention_latent_split(const float* q, const uint16_t* latent_new,
+                                                uint16_t* latent_cache, const int32_t* position,
+                                                int batch, int heads, int latent_dim,
+                                                int max_pos, float scale, float* out,
+                                                void* workspace, hipStream_t s) {
+  if (batch == 0) return hipSuccess;
+  return launch_decode_split<float, float, 0>(q, latent_new, latent_new, latent_cache,
+                                              latent_cache, position, batch, heads, 1, latent_dim,
+                                              max_pos, max_pos, scale, out, HeadsOut{}, workspace,
+                                              s);
 }
 
 }  // namespace parrot

@@ -480,9 +480,11 @@ class LocalGQA(nn.Module):
                 # wraps them (with the addend) in a PendingResidual.
                 return hip_moe.decode_attention_heads(q, k, v, cache.key, cache.value,
                                                       position_device, c.window_size,
-                                                      c.head_dim ** -0.5, self.out.weight)
+                                                      c.head_dim ** -0.5, self.out.weight,
+                                                      context=position + 1)
             y = hip_moe.decode_attention(q, k, v, cache.key, cache.value, position_device,
-                                         c.window_size, c.head_dim ** -0.5)
+                                         c.window_size, c.head_dim ** -0.5,
+                                         context=position + 1)
             width = c.n_heads * c.head_dim
             # The GEMV beats the MFMA projection for one or two rows (measured
             # at b = 1 / 2 / 8: 0.525 -> 0.515, 0.559 -> 0.553, 0.730 -> 0.776 ms
@@ -681,12 +683,12 @@ class GlobalMLA(nn.Module):
                                                          mix=mix)
                 context = hip_moe.decode_attention_latent(
                     q_latent, latent, cache.latent, position_device, c.n_heads,
-                    c.head_dim ** -0.5)
+                    c.head_dim ** -0.5, context=position + 1)
                 return hip_moe.mla_decode_out(context, absorbed_o, addend)
             absorbed_q, absorbed_o = self._absorbed_f32()
             context = hip_moe.decode_attention_latent(
                 F.linear(x.float(), absorbed_q), self.kv_down(x), cache.latent, position_device,
-                c.n_heads, c.head_dim ** -0.5)
+                c.n_heads, c.head_dim ** -0.5, context=position + 1)
             result = F.linear(context.view(b, 1, -1), absorbed_o).to(x.dtype)
             return result if addend is None else addend + result
         absorbed_q, absorbed_o = self._absorbed()

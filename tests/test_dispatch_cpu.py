@@ -1,0 +1,41 @@
+"""Host-side rules that pick a kernel, and the argument checks of their C
+entry points (no GPU)."""
+import ctypes
+
+
+def test_decode_split_rule():
+    from parrot import hip_moe
+    assert not hip_moe.decode_splits(None, 1)
+    assert not hip_moe.decode_splits(352, 1) and hip_moe.decode_splits(353, 1)
+    assert not hip_moe.decode_splits(4096, 1, window=352)  # the window bounds the keys
+    assert not hip_moe.decode_splits(1024, 64) and hip_moe.decode_splits(1025, 64)
+
+
+def test_decode_split_arguments():
+    from parrot import _abi
+    lib, fake, null = _abi.load(), ctypes.c_void_p(4096), None
+    size = lib.parrot_decode_attention_split_workspace_bytes
+    # (max, sum) pairs and partial rows of 32 chunks of 64 keys
+    assert size(1, 8, 2, 96, 4096, 2048) == 8 * 32 * 8 + 8 * 32 * 96 * 4
+    assert size(1, 8, 2, 16, 4096, 2048) == 0 and size(1, 34, 2, 96, 4096, 2048) == 0
+    assert size(1, 8, 3, 96, 4096, 2048) == 0
+
+    def local(q=4096, heads=8, d=96, ws=4096, wsb=1 << 20, out=fake):
+        return lib.parrot_decode_attention_split_bf16(
+            q, fake, fake, fake, fake, fake, 1, heads, 2, d, 4096, 2048, 0.1, out, ws, wsb, null)
+    assert local(q=null) == -1 and local(out=null) == -1
+    assert local(heads=7) == -3 and local(d=16) == -3 and local(heads=34) == -3
+    assert local(ws=null) == -4 and local(wsb=64) == -4
+    assert local(q=4096 + 8) == -5 and local(ws=4096 + 8) == -5
+
+    def heads(dim=768, w=fake, wsb=1 << 20):
+        return lib.parrot_decode_attention_heads_split_bf16(
+            fake, fake, fake, fake, fake, fake, 1, 8, 2, 96, 4096, 2048, 0.1, w, dim, fake, fake,
+            wsb, null)
+    assert heads(w=null) == -1 and heads(dim=0) == -2 and heads(dim=776) == -3
+    assert heads(wsb=64) == -4
+
+    def latent(q=fake, r=128, wsb=1 << 22):
+        return lib.parrot_decode_attention_latent_split_f32(
+            q, fake, fake, fake, 1, 8, r, 4096, 0.1, fake, fake, wsb, null)
+    assert latent(q=null) == -1 and latent(r=100) == -3 and latent(wsb=64) == -4

@@ -1,0 +1,130 @@
+"""GPU parity of the decode attention whose keys are split over workgroups
+(long contexts) with the one-launch form and an fp64 restatement, and of a
+DecodeGraph that crosses from one form to the other."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _split_always(monkeypatch):
+    from parrot import hip_moe
+    monkeypatch.setattr(hip_moe, "decode_splits", lambda context, batch, window=None:
+                        context is not None)
+    return hip_moe
+
+
+def _local_inputs(b, H, Hk, d, max_pos, seed):
+    g = torch.Generator().manual_seed(seed)
+    shapes = ((b, H, 1, d), (b, Hk, 1, d), (b, Hk, 1, d), (b, Hk, max_pos, d),
+              (b, Hk, max_pos, d))
+    return [torch.randn(s, generator=g).bfloat16().cuda() for s in shapes]
+
+
+def _attend64(q, keys, values, scale):
+    """q [b, H, d] over keys / values [b, Hk, L, d], fp64."""
+    rep = q.shape[1] // keys.shape[1]
+    k, v = (t.double().repeat_interleave(rep, 1) for t in (keys, values))
+    s = torch.matmul(k, q.double().unsqueeze(-1)).squeeze(-1) * scale
+    return torch.matmul(s.softmax(-1).unsqueeze(-2), v).squeeze(-2)
+
+
+# chunk edges (64 keys), the window's edge, head groups of 1 to 16, every
+# head width the split form takes, one -inf chunk
+@pytest.mark.parametrize("b,H,Hk,d,max_pos,window,position,masked", [
+    (1, 8, 2, 96, 256, 200, 0, None), (2, 8, 2, 96, 256, 200, 63, None),
+    (1, 8, 2, 96, 256, 200, 64, None), (3, 8, 2, 96, 256, 200, 255, None),
+    (2, 6, 6, 64, 300, 100, 130, None), (1, 16, 1, 128, 700, 700, 699, None),
+    (2, 6, 2, 32, 513, 400, 512, None), (1, 4, 2, 192, 300, 300, 191, None),
+    (1, 2, 1, 256, 300, 300, 299, None), (3, 12, 1, 96, 300, 300, 129, None),
+    (1, 8, 2, 96, 4096, 4096, 4000, None), (1, 8, 2, 96, 300, 300, 250, (64, 128)),
+    (1, 8, 2, 96, 300, 300, 250, (0, 190))])
+def test_split_decode_attention(monkeypatch, b, H, Hk, d, max_pos, window, position, masked):
+    hip_moe = _split_always(monkeypatch)
+    print(f"split decode b={b} H={H}/{Hk} d={d} p={position} window={window}", flush=True)
+    q, kn, vn, kc, vc = _local_inputs(b, H, Hk, d, max_pos, position + d)
+    if masked is not None:  # positive queries against -inf keys: scores of -inf
+        q = q.abs() + 0.125
+        kc[:, :, masked[0]:masked[1]] = float("-inf")
+    pos = torch.tensor([position], dtype=torch.int32, device="cuda")
+    dim, scale = 512, d ** -0.5
+    w = (torch.randn(dim, H * d, device="cuda") * (H * d) ** -0.5).bfloat16()
+    caches = [(kc.clone(), vc.clone()) for _ in range(3)]
+    with torch.no_grad():
+        one = hip_moe.decode_attention(q, kn, vn, *caches[0], pos, window, scale)
+        got = hip_moe.decode_attention(q, kn, vn, *caches[1], pos, window, scale,
+                                       context=position + 1)
+        heads = hip_moe.decode_attention_heads(q, kn, vn, *caches[2], pos, window, scale, w,
+                                               context=position + 1)
+    for k, v in caches:  # the new rows stored, every other row untouched
+        kc[:, :, position], vc[:, :, position] = kn[:, :, 0], vn[:, :, 0]
+        assert torch.equal(k, kc) and torch.equal(v, vc)
+    lo = max(0, position - window + 1)
+    ref = _attend64(q[:, :, 0], kc[:, :, lo:position + 1], vc[:, :, lo:position + 1], scale)
+    got64 = got.double().view(b, H, d)
+    # one bf16 rounding plus fp32 reassociation, as for the one-launch form
+    assert ((got64 - ref).abs() <= 2 ** -8 * ref.abs().max() + 1e-5).all()
+    assert ((one.double().view(b, H, d) - got64).abs() <= 2 ** -7 * ref.abs().max()).all()
+    # each head's contribution: the bf16 output times its weight slice
+    per_head = w.double().view(dim, H, d)
+    want = torch.stack([got64[:, h] @ per_head[:, h].T for h in range(H)], 1)
+    size = torch.stack([got64[:, h].abs() @ per_head[:, h].abs().T for h in range(H)], 1)
+    assert ((heads.double() - want).abs() <= 1e-6 * size + 1e-7).all()
+
+
+@pytest.mark.parametrize("b,H,r,position", [(1, 8, 128, 0), (2, 8, 128, 64), (3, 6, 128, 700),
+                                            (1, 16, 64, 129), (2, 3, 32, 383)])
+def test_split_decode_attention_latent(monkeypatch, b, H, r, position):
+    """fp32 queries (three bf16 parts in the score product) stay fp32 exact:
+    no further from fp64 than the one-launch fp32 dot, within 1e-6."""
+    hip_moe = _split_always(monkeypatch)
+    print(f"split latent b={b} H={H} r={r} p={position}", flush=True)
+    g = torch.Generator().manual_seed(position + r)
+    max_pos = 800
+    q = (torch.randn(b, 1, H * r, generator=g) * 3).cuda()
+    new = torch.randn(b, 1, r, generator=g).bfloat16().cuda()
+    cache = torch.randn(b, max_pos, r, generator=g).bfloat16().cuda()
+    pos = torch.tensor([position], dtype=torch.int32, device="cuda")
+    c1, c2 = cache.clone(), cache.clone()
+    with torch.no_grad():
+        one = hip_moe.decode_attention_latent(q, new, c1, pos, H, 96 ** -0.5)
+        got = hip_moe.decode_attention_latent(q, new, c2, pos, H, 96 ** -0.5,
+                                              context=position + 1)
+    cache[:, position] = new[:, 0]
+    assert torch.equal(c1, cache) and torch.equal(c2, cache)
+    keys = cache[:, None, :position + 1]
+    ref = _attend64(q.view(b, H, r), keys, keys, 96 ** -0.5).view(b, -1)
+    err = [float((x.double() - ref).norm() / ref.norm()) for x in (one, got)]
+    print("  relative error", err, flush=True)
+    assert err[1] <= max(1e-6, 1.5 * err[0])
+
+
+@pytest.mark.parametrize("logits", [False, True])
+def test_decode_graph_crosses_into_the_split_form(logits):
+    """Steps on either side of the position from which the keys are split
+    equal eager steps, and the graph's output stays the same tensor."""
+    from parrot import ModelConfig, Parrot, hip_moe
+    from parrot.decode_graph import DecodeGraph
+    cfg = ModelConfig(vocab_size=512, dim=256, n_layers=4, n_heads=4, n_kv_heads=2, head_dim=64,
+                      kv_latent_dim=64, window_size=512, max_seq_len=512, n_experts=4,
+                      expert_dim=64, shared_expert_dim=64, moe_backend="grouped_hip",
+                      depth_backend="hip", collect_router_stats=False)
+    torch.manual_seed(3)
+    model = Parrot(cfg).to(device="cuda", dtype=torch.bfloat16).eval()
+    first = next(p for p in range(1, 500) if hip_moe.decode_splits(p + 1, 2))
+    prompt = torch.randint(0, 512, (2, first - 2), device="cuda")
+    _, state = model.prefill(prompt)
+    _, eager = model.prefill(prompt)
+    graph = DecodeGraph(model, state, logits=logits)
+    ids, out = prompt[:, -1:].clone(), graph.out
+    for step in range(5):
+        got = graph.step(ids)
+        assert got.data_ptr() == out.data_ptr()
+        want, _ = (model.decode_step if logits else model.decode_next)(ids, eager)
+        assert torch.equal(got, want), f"step {step} at position {eager.position - 1}"
+        ids = (got.argmax(-1) if logits else got).clone()
+    assert set(graph.graphs) == {False, True}
+    with torch.inference_mode():
+        graph._rewind(first - 1)  # back to the one-launch form: no new capture
+    graph.step(ids)
+    assert len(graph.graphs) == 2 and state.position == first
