@@ -32,6 +32,9 @@
 // one), and the partial states (max, sum, O) are merged in wavefront order
 // through LDS at the end.
 //
+// Whole-sequence calls with fragment-order K and V whose grid would not start
+// at once run in attention_tiles.hip instead (see attention_tiles_apply).
+//
 // PROJ: the output projection's share of this head instead of the output
 // itself (the deferred output sum of the reference's decode,
 // parrot/model.py:301-316, applied to whole sequences): the head's rows
@@ -429,11 +432,14 @@ hipError_t launch_causal_attention(const uint16_t* q, const uint16_t* k, const u
                                    int kv_heads, int head_dim, int window, float scale,
                                    uint16_t* out, hipStream_t s) {
   if (batch == 0 || seq == 0) return hipSuccess;
+  const bool frag = k_strides == nullptr;  // fragment-order K and V
+  if (frag && attention_tiles_apply(batch, seq, heads, head_dim, scale))
+    return launch_attention_tiles(q, k, vt, q_strides, batch, seq, heads, kv_heads, head_dim,
+                                  window, scale, out, s);
   AttnArgs a{};
   a.q = q;
   a.k = k;
   a.vt = vt;
-  const bool frag = k_strides == nullptr;  // fragment-order K and V
   for (int i = 0; i < 3; ++i) {
     a.qs[i] = q_strides[i];
     a.ks[i] = frag ? 0 : k_strides[i];

@@ -571,6 +571,13 @@ hipError_t launch_causal_attention(const uint16_t* q, const uint16_t* k, const u
 // with w_out packed as parrot_proj_bf16's weights (n_out rows, heads *
 // head_dim columns).  n_out from attention_out_width_supported.
 bool attention_out_width_supported(int n_out);  // 512, 768, 1024
+// Long sequences (attention_tiles.hip): fragment-order K and V through LDS,
+// shared by the wavefronts of a workgroup.
+bool attention_tiles_apply(int batch, int seq, int heads, int head_dim, float scale);
+hipError_t launch_attention_tiles(const uint16_t* q, const uint16_t* k_frag,
+                                  const uint16_t* v_frag, const int64_t* q_strides, int batch,
+                                  int seq, int heads, int kv_heads, int head_dim, int window,
+                                  float scale, uint16_t* out, hipStream_t s);
 hipError_t launch_causal_attention_out(const uint16_t* q, const uint16_t* k_frag,
                                        const uint16_t* v_frag, const int64_t* q_strides, int batch,
                                        int seq, int heads, int kv_heads, int head_dim, int window,

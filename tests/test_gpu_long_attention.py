@@ -1,0 +1,90 @@
+"""GPU parity of the long-sequence attention (key blocks shared through LDS)
+with the 16-query kernel, which the strided entry runs at every size, and with
+an fp64 restatement."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _reference(q, k, v, scale, window):
+    """fp64 on the GPU, one head at a time: [b, t, H * d]."""
+    b, H, t, d = q.shape
+    rep = H // k.shape[1]
+    i = torch.arange(t, device=q.device)[:, None]
+    j = torch.arange(t, device=q.device)[None, :]
+    hidden = ~((j <= i) & (j > i - window))
+    out = torch.empty(b, t, H, d, dtype=torch.float64, device=q.device)
+    for n in range(b):
+        for h in range(H):
+            s = (q[n, h].double() @ k[n, h // rep].double().T) * scale
+            out[n, :, h] = s.masked_fill(hidden, float("-inf")).softmax(-1) @ v[n, h // rep].double()
+    return out.view(b, t, H * d)
+
+
+def _fragments(hip_moe, k, v):
+    """K and V packed with non-finite padding keys."""
+    t, pad = k.shape[2], hip_moe.key_blocks(k.shape[2]) * 32
+    full = []
+    for x in (k, v):
+        y = torch.full((*x.shape[:2], pad, x.shape[3]), float("nan"), dtype=x.dtype, device="cuda")
+        y[:, :, :t] = x
+        full.append(y)
+    return hip_moe.pack_kv_fragments(*full)
+
+
+# both forms (one and two key groups; the former from 768 tiles of 128 rows),
+# every head width, 1 to 8 query heads per kv head, ragged tails, windows
+# inside a block and longer than the sequence
+@pytest.mark.parametrize("b,H,Hk,t,d,window,scale", [
+    (2, 8, 2, 513, 96, 2048, None), (1, 8, 8, 1025, 96, 4096, None),
+    (2, 8, 2, 1000, 96, 256, None), (9, 6, 6, 161, 64, 33, None),
+    (5, 6, 3, 300, 128, 77, None), (3, 16, 2, 190, 96, 5, None), (2, 9, 3, 490, 64, 490, None),
+    (24, 8, 2, 500, 96, 2048, None), (16, 8, 8, 769, 64, 100, None),
+    (24, 6, 3, 700, 128, 2048, None), (25, 4, 4, 1000, 96, 64, None),
+    (2, 8, 2, 600, 96, 2048, -0.1), (2, 8, 2, 600, 96, 2048, 0.0)])
+def test_long_attention(b, H, Hk, t, d, window, scale):
+    from parrot import hip_moe
+    print(f"long attention b={b} H={H}/{Hk} t={t} d={d} window={window} scale={scale}", flush=True)
+    scale = d ** -0.5 if scale is None else scale
+    g = torch.Generator(device="cuda").manual_seed(t * 7 + d)
+    draw = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()  # noqa: E731
+    q = draw(b, t, H, d).transpose(1, 2)  # rows strided as a projection leaves them
+    k, v = draw(b, Hk, t, d), draw(b, Hk, t, d)
+    kf, vf = _fragments(hip_moe, k, v)
+    with torch.no_grad():
+        got = hip_moe.causal_attention_frag(q, kf, vf, kv_heads=Hk, scale=scale, window=window)
+        old = hip_moe.causal_attention(q, k, v, scale=scale, window=window)
+    ref = _reference(q, k, v, scale, window)
+    err, old_err = (got.double() - ref).abs(), (old.double() - ref).abs()
+    print(f"  max {err.max():.2e} mean {err.mean():.2e}; 16-query kernel max "
+          f"{old_err.max():.2e} mean {old_err.mean():.2e}", flush=True)
+    # P and the output are each rounded to bf16 once, as in the other kernel
+    assert err.mean() <= 1.25 * old_err.mean() + 1e-6
+    assert err.max() <= 1e-2 + 2 ** -7 * ref.abs().max()
+
+
+@pytest.mark.parametrize("b", [2, 24])
+def test_long_attention_non_finite_keys(b):
+    """Scores of -inf weigh nothing; a query that sees no other key is NaN, as
+    in the 16-query kernel; a NaN key poisons the queries that see it only."""
+    from parrot import hip_moe
+    H, Hk, t, d, window = 8, 2, 530, 96, 100
+    g = torch.Generator(device="cuda").manual_seed(b)
+    q = torch.rand(b, H, t, d, generator=g, device="cuda").bfloat16() + 0.125
+    k = torch.randn(b, Hk, t, d, generator=g, device="cuda").bfloat16()
+    v = torch.randn(b, Hk, t, d, generator=g, device="cuda").bfloat16()
+    k[:, :, :40] = float("-inf")
+    k[:, :, 300:350] = float("-inf")
+    k[:, :, 411, 3] = float("nan")
+    kf, vf = _fragments(hip_moe, k, v)
+    with torch.no_grad():
+        got = hip_moe.causal_attention_frag(q, kf, vf, kv_heads=Hk, scale=d ** -0.5, window=window)
+        old = hip_moe.causal_attention(q, k, v, scale=d ** -0.5, window=window)
+    bad = torch.isnan(got)
+    assert torch.equal(bad, torch.isnan(old))
+    rows = bad.any(-1)
+    assert rows[:, :40].all() and not rows[:, 40:411].any()
+    assert rows[:, 411:511].all() and not rows[:, 511:].any()
+    # two roundings to bf16 apart at most (P, then the output)
+    assert (got - old).abs()[~bad].max() <= 2e-2
