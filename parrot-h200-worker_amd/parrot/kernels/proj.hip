@@ -45,6 +45,8 @@
 //             weight (the MLA up-projections).
 #include "common.h"
 
+#include <type_traits>
+
 namespace parrot {
 
 namespace {
@@ -415,6 +417,360 @@ __global__ __launch_bounds__(256) void proj_kernel(ProjArgs p) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Many rows: BM = 32 or 64 rows per workgroup, all of its columns streamed.
+//
+// With 16-row tiles every workgroup pulls its 64 columns' weights (96 KB at
+// K = 768) through L2 for 16 rows: at 16384 rows the q|k|v projection moved
+// 2.3 GB of them and took 128 us, four times its matrix products at the rate
+// of a large library GEMM.  Here the A tile (BM x K, in LDS as above) stays
+// while the wavefronts walk the columns in blocks of 48, each streaming its
+// block's B fragments into a ring of PF register stages that runs on into
+// the wavefront's next block, so the k loop has no barrier and no bubble
+// between blocks; a fragment loaded feeds BM / 16 products.  Measured on
+// MI355X (us, before / now): q|k|v + RoPE with caches 16384 rows 128 / 52
+// (560 TFLOP/s), 4094 rows 36 / 20, 1 x 1024 11.4 / 10.0; output projection
+// with addend 72 / 34, 20 / 12.6; latent q 79 / 34, 23 / 13.5; latent k, v
+// 49 / 22, 15.3 / 9.5.  At 16384 rows each CU runs one workgroup, so its A
+// load, products and stores follow each other; that and the 2-byte stores of
+// row-major values are what is left.
+//
+// The accumulation per output is proj_kernel's (one chain of 16x16x32 MFMAs
+// in k order), so both give the same bits.  Except for attention values the
+// weights are the A operand: lane l then holds row l % 16 of a row tile and
+// four consecutive columns, so RoPE's pairs sit in one lane and every store
+// is 8 bytes.  Values keep x as the A operand (four consecutive positions of
+// one column, what the fragment order wants).  RoPE's cos / sin rows are
+// staged in LDS once for all heads.
+constexpr int kBlockGroups = 3;             // 16-column groups per block
+constexpr int kBlockCols = 16 * kBlockGroups;
+
+// The columns as blocks: [0, n_swap) with the weights as the A operand, then
+// [n_swap, N) with x (no block holds both).
+struct ColumnBlocks {
+  int n_swap, first, total;  // first: blocks of [0, n_swap)
+};
+
+__device__ __forceinline__ ColumnBlocks column_blocks(int n_swap, int N) {
+  const int first = (n_swap + kBlockCols - 1) / kBlockCols;
+  return ColumnBlocks{n_swap, first, first + (N - n_swap + kBlockCols - 1) / kBlockCols};
+}
+
+// One workgroup per CU (98 KB of A at BM = 64; two wavefronts per SIMD).
+template <int BM, int NW, int KST, int EPI>
+__global__ __launch_bounds__(64 * NW, 2) void proj_rows_kernel(ProjArgs p, int splits) {
+  constexpr int kTilesM = BM / 16;
+  constexpr int K = 32 * KST;
+  constexpr int kChunks = K / 8;       // 16-byte chunks per row (a multiple of 16)
+  constexpr int PF = 4;
+  static_assert(KST % PF == 0 && kChunks % 16 == 0, "whole rings, 16-chunk swizzle");
+  __shared__ __attribute__((aligned(16))) uint16_t a_s[BM * K];
+  // (cos, sin) of the tile's rows, d / 2 pairs each (d <= 128)
+  __shared__ __attribute__((aligned(16))) float2 rope_s[EPI == kRopeQkv ? BM * 64 : 1];
+
+  asm volatile("" ::"s"(p.x), "s"(p.lda), "s"(p.rows), "s"(p.N), "s"(p.w), "s"(splits),
+               "s"(p.seq), "s"(p.head_dim));
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, c = lane & 15;
+  const int row_tile = static_cast<int>(blockIdx.x) / splits;
+  const int split = static_cast<int>(blockIdx.x) - row_tile * splits;
+  // Outputs laid out per sequence take row tiles of one sequence each, so a
+  // tile's positions start at a multiple of 4 whatever the length.
+  int b = 0, t0 = row_tile * BM, seq = p.rows;
+  if constexpr (EPI != kStore) {
+    const int per_seq = (p.seq + BM - 1) / BM;
+    b = row_tile / per_seq;
+    t0 = (row_tile - b * per_seq) * BM;
+    seq = p.seq;
+  }
+  const int m0 = b * p.seq + t0;  // first row (b is 0 with plain rows)
+  const int tile_rows = min(BM, seq - t0);
+  const int d = p.head_dim;
+  const int n_swap = EPI == kRopeQkv ? (p.heads + p.kv_heads) * d
+                     : EPI == kFrag  ? (p.kf == nullptr ? 0 : p.vf == nullptr ? p.N : p.N / 2)
+                                     : p.N;
+  const ColumnBlocks cb = column_blocks(n_swap, p.N);
+  const int blk_end = (split + 1) * cb.total / splits;
+  int blk = split * cb.total / splits + wave;
+
+  // ---- A: the whole tile, direct to LDS (rows past the end read the last row)
+  {
+    const __amdgpu_buffer_rsrc_t x_rsrc =
+        make_rsrc(p.x + static_cast<int64_t>(m0) * p.lda,
+                  static_cast<uint32_t>(static_cast<int64_t>(tile_rows) * p.lda * 2));
+    for (int i = wave; i < BM * kChunks / kWave; i += NW) {
+      const int s = i * kWave + lane;
+      const int r = s / kChunks;
+      const int pc = s - r * kChunks;
+      const int ch = (pc & ~15) | ((pc ^ r) & 15);
+      const uint32_t off =
+          static_cast<uint32_t>((static_cast<int64_t>(min(r, tile_rows - 1)) * p.lda + ch * 8) * 2);
+      buffer_to_lds16(x_rsrc, a_s + i * kWave * 8, off, 0);
+    }
+  }
+  if constexpr (EPI == kRopeQkv) {
+    const int half = d / 2;
+    const int shift = p.start + (p.start_device != nullptr ? *p.start_device : 0);
+    for (int i = tid; i < BM * half; i += 64 * NW) {
+      const int r = i / half;
+      const int pos = min(max(shift + t0 + r, 0), p.max_positions - 1);
+      const int64_t at = static_cast<int64_t>(pos) * half + (i - r * half);
+      rope_s[i] = make_float2(p.cos_t[at], p.sin_t[at]);
+    }
+  }
+
+  // Column block b: first column and 16-column groups (uniform).
+  auto first_col = [&](int b) {
+    return b < cb.first ? b * kBlockCols : cb.n_swap + (b - cb.first) * kBlockCols;
+  };
+  const __amdgpu_buffer_rsrc_t b_rsrc =
+      make_rsrc(p.w, static_cast<uint32_t>(static_cast<int64_t>(p.N) * K * 2));
+  uint4 bq[PF][kBlockGroups];
+  // Step `step` of the block whose first column is col0 (columns past N read 0).
+  auto load_step = [&](uint4 (&dst)[kBlockGroups], int col0, int step) {
+#pragma unroll
+    for (int j = 0; j < kBlockGroups; ++j)
+      dst[j] = buffer_load16(b_rsrc, lane * 16u,
+                             static_cast<uint32_t>((col0 / 16 + j) * KST + step) * 1024u);
+  };
+  const int col_first = first_col(min(blk, cb.total - 1));
+#pragma unroll
+  for (int i = 0; i < PF; ++i) load_step(bq[i], col_first, i);
+
+  // A fragment of k step 4 n + q, row tile mi: element a_off[q] + 128 n +
+  // 16 K mi (chunk 4 q + g of the row, swizzled within its group of 16).
+  int a_off[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) a_off[q] = c * K + ((4 * q + g) ^ c) * 8;
+
+  __syncthreads();
+  bf16x8 af[2][kTilesM];
+  auto read_a = [&](bf16x8 (&dst)[kTilesM], int q, int step) {  // q = step % 4
+#pragma unroll
+    for (int mi = 0; mi < kTilesM; ++mi)
+      dst[mi] = *reinterpret_cast<const bf16x8*>(a_s + a_off[q] + (step >> 2) * 128 + mi * 16 * K);
+  };
+  read_a(af[0], 0, 0);
+
+  auto run_block = [&](auto swap_tag, int col0, int next_col0) {
+    constexpr bool SWAP = decltype(swap_tag)::value;
+    const int n_end = SWAP ? cb.n_swap : p.N;  // stores stop at the range's end
+    uint2 add_v[EPI == kStore ? kTilesM : 1][kBlockGroups];
+    if constexpr (EPI == kStore) {
+      // loaded before the products, unconditionally (see proj_kernel)
+      const bool has = p.addend != nullptr;
+      const uint16_t* ab = has ? p.addend : p.w;
+      const int64_t ald = has ? p.ld_addend : 0;
+#pragma unroll
+      for (int mi = 0; mi < kTilesM; ++mi)
+#pragma unroll
+        for (int j = 0; j < kBlockGroups; ++j) {
+          const int row = m0 + min(mi * 16 + c, tile_rows - 1);
+          const int col = min(col0 + 16 * j, p.N - 16) + 4 * g;
+          add_v[mi][j] = *reinterpret_cast<const uint2*>(ab + static_cast<int64_t>(row) * ald + col);
+        }
+    }
+    f32x4 acc[kTilesM][kBlockGroups];
+#pragma unroll
+    for (int mi = 0; mi < kTilesM; ++mi)
+#pragma unroll
+      for (int j = 0; j < kBlockGroups; ++j) acc[mi][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1  // the ring's registers are indexed by i alone
+    for (int s0 = 0; s0 < KST; s0 += PF) {
+#pragma unroll
+      for (int i = 0; i < PF; ++i) {
+        const int step = s0 + i;
+        const int ahead = step + 1 < KST ? step + 1 : 0;  // A fragments, one step ahead
+        read_a(af[(i + 1) & 1], (i + 1) & 3, ahead);
+#pragma unroll
+        for (int mi = 0; mi < kTilesM; ++mi)
+#pragma unroll
+          for (int j = 0; j < kBlockGroups; ++j) {
+            const bf16x8 bf = __builtin_bit_cast(bf16x8, bq[i][j]);
+            acc[mi][j] =
+                SWAP ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf, af[i & 1][mi], acc[mi][j], 0, 0, 0)
+                     : __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i & 1][mi], bf, acc[mi][j], 0, 0, 0);
+          }
+        // the slot's refill: this block's step + PF, or the next block's start
+        const bool more = s0 + PF < KST;
+        load_step(bq[i], more ? col0 : next_col0, more ? step + PF : i);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+
+    // The tile's first position enters the addresses below afresh for every
+    // block: hoisted out of the loop over blocks, those would hold dozens of
+    // registers.
+    int ta = t0;
+    asm volatile("" : "+s"(ta));
+#pragma unroll
+    for (int j = 0; j < kBlockGroups; ++j) {
+      const int nw = col0 + 16 * j;  // uniform
+      if (nw >= n_end) continue;
+      if constexpr (EPI == kStore) {
+#pragma unroll
+        for (int mi = 0; mi < kTilesM; ++mi) {
+          const int row = ta + mi * 16 + c;
+          if (row >= seq) continue;
+          uint16_t v[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = f32_to_bf16(acc[mi][j][r]);
+          if (p.addend != nullptr) {
+            const uint2 a = add_v[mi][j];
+            v[0] = f32_to_bf16(lo_bf16(a.x) + bf16_to_f32(v[0]));
+            v[1] = f32_to_bf16(hi_bf16(a.x) + bf16_to_f32(v[1]));
+            v[2] = f32_to_bf16(lo_bf16(a.y) + bf16_to_f32(v[2]));
+            v[3] = f32_to_bf16(hi_bf16(a.y) + bf16_to_f32(v[3]));
+          }
+          *reinterpret_cast<uint2*>(p.out + static_cast<int64_t>(row) * p.ldo + nw + 4 * g) =
+              make_uint2(v[0] | static_cast<uint32_t>(v[1]) << 16, v[2] | static_cast<uint32_t>(v[3]) << 16);
+        }
+      } else if constexpr (SWAP) {
+        // queries and keys (kRopeQkv, rotated) or keys (kFrag): one head per group
+        const int head = nw / d;
+        const int w = nw - head * d + 4 * g;
+        const int H = EPI == kRopeQkv ? p.heads : 0;
+        const int Hk = EPI == kRopeQkv ? p.kv_heads : n_swap / d;
+#pragma unroll
+        for (int mi = 0; mi < kTilesM; ++mi) {
+          float x[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) x[r] = bf16_round(acc[mi][j][r]);
+          if constexpr (EPI == kRopeQkv) {
+            const float4 cs = *reinterpret_cast<const float4*>(&rope_s[(mi * 16 + c) * (d / 2) + w / 2]);
+            const float e0 = x[0], o0 = x[1], e1 = x[2], o1 = x[3];
+            x[0] = rope_even(e0, o0, cs.x, cs.y);
+            x[1] = rope_odd(e0, o0, cs.x, cs.y);
+            x[2] = rope_even(e1, o1, cs.z, cs.w);
+            x[3] = rope_odd(e1, o1, cs.z, cs.w);
+          }
+          const int t = ta + mi * 16 + c;
+          if (t >= seq) continue;
+          const uint2 v = make_uint2(pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3]));
+          if (head < H) {
+            *reinterpret_cast<uint2*>(
+                p.q + ((static_cast<int64_t>(b) * H + head) * seq + t) * d + w) = v;
+          } else {
+            const int64_t bh = static_cast<int64_t>(b) * Hk + head - H;
+            if (EPI == kRopeQkv && p.k != nullptr)
+              *reinterpret_cast<uint2*>(p.k + (bh * seq + t) * d + w) = v;
+            if (p.kf != nullptr)
+              *reinterpret_cast<uint2*>(p.kf + kfrag_index(bh, p.nblk, t, w, d / 32)) = v;
+          }
+        }
+      } else {
+        // values: lane holds column c, positions t .. t + 3 (t % 4 == 0)
+        const int head = (nw - n_swap) / d;
+        const int w = nw - n_swap - head * d + c;
+        const int Hv = EPI == kRopeQkv ? p.kv_heads : (p.N - n_swap) / d;
+        const int64_t bh = static_cast<int64_t>(b) * Hv + head;
+#pragma unroll
+        for (int mi = 0; mi < kTilesM; ++mi) {
+          const int t = ta + mi * 16 + 4 * g;
+          if (t >= seq) continue;
+          uint16_t bits[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) bits[r] = f32_to_bf16(acc[mi][j][r]);
+          const uint2 v = make_uint2(bits[0] | static_cast<uint32_t>(bits[1]) << 16,
+                                     bits[2] | static_cast<uint32_t>(bits[3]) << 16);
+          // (positions past the sequence fall on the last block's padding keys)
+          if (p.vf != nullptr)
+            *reinterpret_cast<uint2*>(p.vf + vfrag_index(bh, p.nblk, t, w, d / 16)) = v;
+          if (EPI == kRopeQkv && p.v != nullptr) {
+            if (p.ld_keys > 0 && t + 4 <= seq) {
+              *reinterpret_cast<uint2*>(p.v + (bh * d + w) * p.ld_keys + t) = v;
+            } else {
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                if (t + r < seq)
+                  p.v[p.ld_keys > 0 ? (bh * d + w) * p.ld_keys + t + r : (bh * seq + t + r) * d + w] =
+                      bits[r];
+            }
+          }
+        }
+      }
+    }
+  };
+
+  for (; blk < blk_end; blk += NW) {
+    const int col0 = first_col(blk);
+    const int next = first_col(min(blk + NW, cb.total - 1));
+    if (blk < cb.first) run_block(std::true_type{}, col0, next);
+    else run_block(std::false_type{}, col0, next);
+  }
+}
+
+// Row tiles of bm rows, of one sequence each where the outputs are laid out
+// per sequence.
+template <int EPI>
+int row_tiles(const ProjArgs& a, int bm) {
+  if (EPI == kStore) return (a.rows + bm - 1) / bm;
+  return a.rows / a.seq * ((a.seq + bm - 1) / bm);
+}
+
+// BM = 32 up to 4096 rows, where 64-row tiles leave a wavefront one block of
+// columns and the A tile's load stands out (2 x 2047 rows: q|k|v 22.0 -> 19.8
+// us, output 15.3 -> 12.6 us); 64 beyond, for half the weight traffic (2 x
+// 4096: 35.7 -> 31.3 and 22.9 -> 20.7 us).
+constexpr int kRows32 = 4096;
+// From where the tiles beat proj_kernel (16 x 64 per workgroup; us, that
+// kernel / this): q|k|v 768 rows 9.7 / 9.5, 999 rows 11.7 / 9.5; values and
+// keys from the latent 768 rows 5.3 / 5.3, 999 rows 6.6 / 5.9; the plain
+// output 999 rows 7.1 / 7.3, 1024 rows 7.2 / 7.4, 1500 rows 9.7 / 8.4.
+constexpr int kRowsFrom = 960, kStoreRowsFrom = 1100;
+
+template <int EPI>
+bool rows_apply(const ProjArgs& a) {
+  const int steps = a.K / 32;
+  if (a.K % 32 || (steps != 4 && steps != 8 && steps != 16 && steps != 24)) return false;
+  // 8-byte accesses of the row-major operands and outputs
+  const auto aligned8 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; };
+  if (EPI == kStore)
+    return a.rows >= kStoreRowsFrom && a.ldo % 4 == 0 && aligned8(a.out) &&
+           (a.addend == nullptr || (a.ld_addend % 4 == 0 && aligned8(a.addend)));
+  // whole heads per 16-column group; sequences of at least four tiles, so that
+  // their ragged ends stay a small part
+  const int bm = a.rows <= kRows32 ? 32 : 64;
+  return a.rows >= kRowsFrom && a.seq >= 4 * bm && a.head_dim % 16 == 0 && a.head_dim <= 128 &&
+         a.ld_keys % 4 == 0 && aligned8(a.q) && aligned8(a.k) && aligned8(a.v) && aligned8(a.kf) &&
+         aligned8(a.vf);
+}
+
+template <int BM, int EPI>
+hipError_t launch_rows(const ProjArgs& a, hipStream_t s) {
+  constexpr int NW = 8;
+  const int tiles = row_tiles<EPI>(a, BM);
+  // Column splits, each with its own copy of the A tile: the fewest rounds of
+  // one workgroup per CU times what one takes (in column blocks of a
+  // wavefront: about one for the A tile and the start, its blocks, and a tenth
+  // for every block of the workgroup, whose wavefronts share the CU).
+  const int blocks = (a.N + kBlockCols - 1) / kBlockCols;
+  int splits = 1;
+  float best = 0.0f;
+  for (int n = 1; n <= 8 && n <= blocks; ++n) {
+    const int64_t rounds = (static_cast<int64_t>(tiles) * n + 255) / 256;
+    const int per_group = (blocks + n - 1) / n;
+    const int per_wave = (per_group + NW - 1) / NW;
+    const float cost = static_cast<float>(rounds) *
+                       (1.0f + static_cast<float>(per_wave) + 0.1f * static_cast<float>(per_group));
+    if (n == 1 || cost < best) {
+      splits = n;
+      best = cost;
+    }
+  }
+  const int grid = tiles * splits;
+  switch (a.K / 32) {
+    case 4: proj_rows_kernel<BM, NW, 4, EPI><<<grid, 64 * NW, 0, s>>>(a, splits); break;
+    case 8: proj_rows_kernel<BM, NW, 8, EPI><<<grid, 64 * NW, 0, s>>>(a, splits); break;
+    case 16: proj_rows_kernel<BM, NW, 16, EPI><<<grid, 64 * NW, 0, s>>>(a, splits); break;
+    case 24: proj_rows_kernel<BM, NW, 24, EPI><<<grid, 64 * NW, 0, s>>>(a, splits); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
 int ring_depth(int ksteps) {
   for (int pf = 8; pf > 1; pf >>= 1)
     if (ksteps % pf == 0) return pf;
@@ -424,6 +780,10 @@ int ring_depth(int ksteps) {
 template <int EPI>
 hipError_t launch_proj(const ProjArgs& a, hipStream_t s) {
   if (a.rows == 0 || a.N == 0) return hipSuccess;
+  if constexpr (EPI != kStoreT) {
+    if (rows_apply<EPI>(a))
+      return a.rows <= kRows32 ? launch_rows<32, EPI>(a, s) : launch_rows<64, EPI>(a, s);
+  }
   const int tiles = ((a.rows + kProjRows - 1) / kProjRows) * ((a.N + kProjCols - 1) / kProjCols);
   const size_t lds = static_cast<size_t>(kProjRows) * a.K * 2;
   switch (a.K / 32) {
