@@ -27,6 +27,7 @@ constexpr uint32_t kNoExpert = 0xff;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // A streaming store of 4 bf16: the nt hint keeps a long output's lines from
 // displacing cached inputs and lets HBM take the writes in larger bursts.

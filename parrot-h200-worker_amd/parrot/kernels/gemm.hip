@@ -25,6 +25,7 @@
 // to assignment order (fp32), shared rows go to token order (fp32).
 #include "common.h"
 
+
 namespace parrot {
 
 namespace {
@@ -685,18 +686,14 @@ void grouped_gemm_kernel(GemmArgs p) {
 }
 
 // ---------------------------------------------------------------------------
-// Wide-MFMA tiles for large segments (hundreds to thousands of rows per
-// expert): the same LDS ring as grouped_gemm_kernel (direct-to-LDS stages of
+// Wide-MFMA tiles for large segments whose k loops are too short for the
+// persistent kernel below: the same LDS ring as grouped_gemm_kernel (direct-to-LDS stages of
 // 1 KB fragment-order blocks, BK = 64, one barrier per k step), with a
 // 128 x 128 workgroup tile computed on v_mfma_f32_32x32x16_bf16.  Measured
 // on MI355X, that MFMA keeps 92 % of the bf16 peak issuing from one
 // wavefront per SIMD where 16x16x32 keeps 70 %, and a 64 x 64 wavefront
 // tile reads 4 fragments from LDS per 4 MFMAs of 32 K flops each.
-// WAVES_M x WAVES_N wavefronts share the tile: 2 x 2 for 128 x 128 tiles
-// (64 x 64 per wavefront), 2 x 4 for 256 x 256 ones (128 x 64 per wavefront:
-// 6 fragment reads per 8 MFMAs, and half the stage bytes per flop, at one
-// workgroup per CU).  The 256 x 256 tile's route weights go through LDS:
-// its 128 accumulators per lane leave no registers for them.
+// Four wavefronts (2 x 2) share the tile.
 //
 // 32x32x16 operands: lane l holds row (or column) l % 32, k 8 (l / 32) .. +7
 // of a 16-wide k step.  In the 16 x 32 fragment-order blocks that is block
@@ -706,9 +703,10 @@ void grouped_gemm_kernel(GemmArgs p) {
 // 8 (e / 4) + 4 (l / 32) + e % 4 of element e.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-template <int BM, int BN, int BK, int S, int PHASE, int WAVES_M = 2, int WAVES_N = 2>
-__global__ __launch_bounds__(64 * WAVES_M * WAVES_N)
+template <int BM, int BN, int BK, int S, int PHASE>
+__global__ __launch_bounds__(256)
 void grouped_gemm_wide_kernel(GemmArgs p) {
+  constexpr int WAVES_M = 2, WAVES_N = 2;
   constexpr int kWaves = WAVES_M * WAVES_N;
   constexpr int kThreads = 64 * kWaves;
   constexpr int kWaveM = BM / WAVES_M, kWaveN = BN / WAVES_N;  // wavefront tile
@@ -727,10 +725,6 @@ void grouped_gemm_wide_kernel(GemmArgs p) {
   __shared__ __attribute__((aligned(16))) uint16_t ring[S][kStageElems];
   __shared__ int row_src[BM];
   __shared__ int row_dst[BM];
-  // Route weights of the tile's rows, for wavefront tiles whose registers
-  // cannot also hold them (kRouteInLds).
-  constexpr bool kRouteInLds = kTilesM * kTilesN * 16 > 64;
-  __shared__ float row_w[kRouteInLds ? BM : 1];
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -768,7 +762,6 @@ void grouped_gemm_wide_kernel(GemmArgs p) {
     row_src[tid] = PHASE == 1 ? (shared ? sc : asg >> 1) : t.hbase + sc;
     const bool live = t.mt * BM + tid < t.rows;
     row_dst[tid] = !live ? -1 : PHASE == 1 ? t.hbase + sc : (shared ? sc : asg);
-    if (kRouteInLds && PHASE == 2) row_w[tid] = live && !shared ? p.weights[asg] : 0.0f;
   }
   __syncthreads();
 
@@ -835,8 +828,8 @@ void grouped_gemm_wide_kernel(GemmArgs p) {
 
   // Route weights of this lane's output rows (phase 2, routed): issued here,
   // they land while the k loop runs instead of stalling the epilogue.
-  float route_w[kRouteInLds ? 1 : kTilesM][16];
-  if (!kRouteInLds && PHASE == 2 && !shared) {
+  float route_w[kTilesM][16];
+  if (PHASE == 2 && !shared) {
 #pragma unroll
     for (int i = 0; i < kTilesM; ++i)
 #pragma unroll
@@ -938,14 +931,412 @@ void grouped_gemm_wide_kernel(GemmArgs p) {
           const int row = wm0 + 32 * i + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
           const int dst = row_dst[row];
           const int64_t at = static_cast<int64_t>(max(dst, 0)) * p.dim + n;
-          const float w = shared ? 1.0f
-                                 : (kRouteInLds ? row_w[row] : route_w[kRouteInLds ? 0 : i][e]);
-          const float v = shared ? acc[i][j][e] : w * acc[i][j][e];
+          const float v = shared ? acc[i][j][e] : route_w[i][e] * acc[i][j][e];
           if (dst >= 0 && n < N) (shared ? p.y_shared : p.y_routed)[at] = f32_to_bf16(v);
         }
       }
     }
   }
+}
+
+// ---------------------------------------------------------------------------
+// Persistent 128 x 256 tiles for segments of hundreds of rows and more.
+//
+// Two workgroups per CU (four wavefronts each, 128 rows x 64 columns per
+// wavefront) walk their XCD's list of tiles, and the pipeline of stages runs
+// on from tile to tile: while a tile's last stages are computed and its
+// outputs stored, the next tile's row ids, then its first stages, are already
+// on their way.  The one-tile-per-workgroup kernel spends as long on that
+// chain (counts -> row ids -> first stage) and on its epilogue as on the 24
+// (or 16) k steps of a tile; and with two independent workgroups on a CU one
+// multiplies while the other waits, applies SwiGLU or stores.
+//
+//   stages    32 k values of A (128 gathered rows) and B (256 packed weight
+//             rows), 24 KB, direct to LDS in a ring of three.
+//   products  v_mfma_f32_32x32x16_bf16 with the weights as the A operand: a
+//             lane then holds one token row of each 32-row tile and, of every
+//             32 packed gate / up rows, 8 gate values and their 8 up values,
+//             so SwiGLU needs no exchange and a lane needs one route weight per
+//             32-row tile.  Rows leave through the stage buffer just read, as
+//             64-byte runs.
+//   row ids   direct to LDS too (one dword copy per row), so nothing in the
+//             loop waits for a register load.
+//
+// Waits: every wavefront issues kCopies copies per stage; stage kt has landed
+// when at most those of stage kt + 1 are outstanding.  Stages 0 and 1 of a
+// tile were issued before the previous tile's kStores stores, which may be
+// outstanding as well (vector-memory operations retire in order).  Row id and
+// route weight copies only make those waits stricter.  A tile needs 7 k steps
+// for its successor's row ids and its own route weights to land in time
+// (kBigKMin asks for 8).
+//
+// Bound by the matrix cores together with what the wavefronts issue beside
+// them: with 256 x 256 tiles, of gate/up's 157 us at 32768 tokens, leaving out
+// the products, the copies or the LDS reads saved 15-20 us each, the epilogue
+// 35.  Measured on MI355X at 32768 tokens, 16 experts (a graph of 10
+// launches, 128 x 128 tiles of one workgroup each / this): gate/up 211 /
+// 147 us (1.05 PFLOP/s), down 133 / 89 us.  65536 tokens: 373 / 281 and
+// 276 / 204.  16384: 119 / 85 and 76 / 49.  256 x 256 tiles in one workgroup of
+// eight wavefronts per CU, in step or half a stage apart: 157-166 and 92-97.
+// Copies issued after a stage's first products instead of before: 168 -> 162.
+constexpr int kBigRows = 128;
+constexpr int kBigCols = 256;
+constexpr int kBigK = 32;       // k values per stage
+constexpr int kBigStages = 3;
+constexpr int kBigKMin = 8 * kBigK;
+
+// One 16-wide k step's six fragments from LDS, landed on return: token rows at
+// `t` + 2048 i + O, weight rows at `w` + 2048 j + O (one asm block: no register
+// is named before its data is there, and the compiler ties nothing to the
+// copies in flight).
+template <int O>
+__device__ __forceinline__ void read_step6(uint32_t t, uint32_t w, bf16x8 (&a)[4], bf16x8 (&b)[2]) {
+  asm volatile(
+      "ds_read_b128 %4, %7 offset:%8\n\tds_read_b128 %0, %6 offset:%8\n\t"
+      "ds_read_b128 %5, %7 offset:%9\n\tds_read_b128 %1, %6 offset:%9\n\t"
+      "ds_read_b128 %2, %6 offset:%10\n\tds_read_b128 %3, %6 offset:%11\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2]), "=&v"(a[3]), "=&v"(b[0]), "=&v"(b[1])
+      : "v"(t), "v"(w), "i"(O), "i"(O + 2048), "i"(O + 4096), "i"(O + 6144));
+}
+
+__device__ __forceinline__ void join() { asm volatile("s_barrier" ::: "memory"); }
+
+template <int N>
+__device__ __forceinline__ void copies_left() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
+}
+
+// A wavefront's 32 rows x 32 bf16 values through its own LDS rows (kOutLd
+// values apart): lane l brings values 8 q + 4 (l / 32) .. + 3 of row l % 32 as
+// v[q] and leaves with values 8 (l % 4) .. + 7 of rows l / 4 and 16 + l / 4,
+// so that a row is stored as one 64-byte run instead of eight 8-byte pieces
+// (one block of asm: a compiler-made LDS access would wait for the copies in
+// flight).
+constexpr int kOutLd = 40;
+
+__device__ __forceinline__ void rows_through_lds(uint32_t base, const u32x2 (&v)[4], u32x4 (&o)[2]) {
+  const uint32_t lane = threadIdx.x & (kWave - 1);
+  const uint32_t wr = base + (lane & 31) * (kOutLd * 2) + (lane >> 5) * 8;
+  const uint32_t rd = base + (lane >> 2) * (kOutLd * 2) + (lane & 3) * 16;
+  asm volatile(
+      "ds_write_b64 %2, %4\n\tds_write_b64 %2, %5 offset:16\n\t"
+      "ds_write_b64 %2, %6 offset:32\n\tds_write_b64 %2, %7 offset:48\n\t"
+      "ds_read_b128 %0, %3\n\tds_read_b128 %1, %3 offset:%8\n\ts_waitcnt lgkmcnt(0)"
+      : "=&v"(o[0]), "=&v"(o[1])
+      : "v"(wr), "v"(rd), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "i"(16 * kOutLd * 2));
+}
+
+// Eight dwords from LDS at addr + 64 i, landed on return.
+__device__ __forceinline__ void read_dwords8(uint32_t addr, int (&v)[8]) {
+  asm volatile(
+      "ds_read_b32 %0, %8\n\tds_read_b32 %1, %8 offset:64\n\tds_read_b32 %2, %8 offset:128\n\t"
+      "ds_read_b32 %3, %8 offset:192\n\tds_read_b32 %4, %8 offset:256\n\t"
+      "ds_read_b32 %5, %8 offset:320\n\tds_read_b32 %6, %8 offset:384\n\t"
+      "ds_read_b32 %7, %8 offset:448\n\ts_waitcnt lgkmcnt(0)"
+      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]),
+        "=&v"(v[7])
+      : "v"(addr));
+}
+
+// Four dwords from LDS at addr + 128 i, landed on return.
+__device__ __forceinline__ void read_dwords4(uint32_t addr, int (&v)[4]) {
+  asm volatile(
+      "ds_read_b32 %0, %4\n\tds_read_b32 %1, %4 offset:128\n\tds_read_b32 %2, %4 offset:256\n\t"
+      "ds_read_b32 %3, %4 offset:384\n\ts_waitcnt lgkmcnt(0)"
+      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])
+      : "v"(addr));
+}
+
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+  return static_cast<uint32_t>(
+      reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)p));
+}
+
+__device__ __forceinline__ void buffer_to_lds4(__amdgpu_buffer_rsrc_t r, void* lds,
+                                               uint32_t voffset) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void_t*)lds, 4, voffset, 0, 0, 0);
+}
+
+template <int PHASE>
+__global__ __launch_bounds__(256, 2) void grouped_gemm_big_kernel(GemmArgs p) {
+  constexpr int kStageElems = (kBigRows + kBigCols) * kBigK;
+  constexpr int kCopies = 6;  // per wavefront and stage
+  constexpr int kStores = PHASE == 1 ? 8 : 16;  // per wavefront and tile, always issued
+  __shared__ __attribute__((aligned(16))) uint16_t ring[kBigStages][kStageElems];
+  __shared__ int ids_s[2][kBigRows];   // assignment ids of the routed rows, by tile parity
+  __shared__ int w_s[kBigRows];        // their route weights (phase 2)
+
+  load_gemm_args(p);
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int T = static_cast<int>(p.tokens);
+  const int E = p.experts;
+
+  // Lane e: expert e's rows, tiles and offsets.
+  const bool mine = lane < E;
+  const int count = mine ? p.counts[lane] : 0;
+  const int hoff = mine ? p.offsets[lane] : 0;
+  const int ooff = mine ? p.offsets[E + 1 + lane] : 0;
+  const int tiles = (count + kBigRows - 1) / kBigRows;
+  const int tile_end = scan32(tiles);
+  const int tile0 = tile_end - tiles;
+  const int routed_m = __builtin_amdgcn_readlane(tile_end, E - 1);
+  const int shared_m = (T + kBigRows - 1) / kBigRows;
+  const int Nr = PHASE == 1 ? 2 * p.hidden_dim : p.dim;
+  const int Ns = PHASE == 1 ? 2 * p.shared_dim : p.dim;
+  const int nr = (Nr + kBigCols - 1) / kBigCols, ns = (Ns + kBigCols - 1) / kBigCols;
+
+  // This XCD's tiles: row tiles x, x + 8, ... with all their column tiles in
+  // turn, the routed ones first; this workgroup takes every gridDim / 8-th.
+  const int xcd = static_cast<int>(blockIdx.x) & 7;
+  const int list_r = ((routed_m + 7 - xcd) >> 3) * nr;
+  const int list_all = list_r + ((shared_m + 7 - xcd) >> 3) * ns;
+  const int step = static_cast<int>(gridDim.x) >> 3;
+
+  struct Work {
+    Tile t;
+    int n0, N, K;
+  };
+  auto locate = [&](int i) {
+    Work w;
+    if (i < list_r) {
+      const int q = i / nr;
+      const int m = xcd + 8 * q;
+      const uint64_t hit = __ballot(mine && m >= tile0 && m < tile_end);
+      const int seg = static_cast<int>(__builtin_ctzll(hit));
+      w.t = Tile{seg, m - __builtin_amdgcn_readlane(tile0, seg),
+                 __builtin_amdgcn_readlane(count, seg), __builtin_amdgcn_readlane(hoff, seg),
+                 __builtin_amdgcn_readlane(ooff, seg)};
+      w.n0 = (i - q * nr) * kBigCols;
+      w.N = Nr;
+      w.K = PHASE == 1 ? p.dim : p.hidden_dim;
+    } else {
+      const int q = (i - list_r) / ns;
+      w.t = Tile{E, xcd + 8 * q, T, 2 * T, 0};
+      w.n0 = (i - list_r - q * ns) * kBigCols;
+      w.N = Ns;
+      w.K = PHASE == 1 ? p.dim : p.shared_dim;
+    }
+    w.t = uniform_tile(w.t);
+    w.n0 = __builtin_amdgcn_readfirstlane(w.n0);
+    return w;
+  };
+
+  // Row ids of a routed tile into ids_s[buf] (wavefronts 0 and 1, one row per lane).
+  auto load_ids = [&](const Work& w, int buf) {
+    if (w.t.seg == E || wave >= kBigRows / kWave) return;
+    const int s = w.t.mt * kBigRows + tid;
+    int* dst = &ids_s[buf][wave * kWave];
+    if (s >= w.t.rows) return;
+    if (p.sorted != nullptr) {
+      buffer_to_lds4(make_rsrc(p.sorted, static_cast<uint32_t>(T) * 8u), dst,
+                     static_cast<uint32_t>(w.t.hbase + s) * 4u);
+    } else if (s < p.capacity) {
+      buffer_to_lds4(make_rsrc(p.perm, static_cast<uint32_t>(E) * p.capacity * 4u), dst,
+                     static_cast<uint32_t>(w.t.seg * p.capacity + s) * 4u);
+    } else {
+      buffer_to_lds4(make_rsrc(p.overflow, static_cast<uint32_t>(T) * 8u), dst,
+                     static_cast<uint32_t>(w.t.obase + s - p.capacity) * 4u);
+    }
+  };
+
+  // Copy state: each wavefront copies two of a stage's eight 1 KB blocks of A
+  // (16 rows x 32 k values) and four of its sixteen blocks of B.
+  const int a_ld = PHASE == 1 ? p.dim : p.hstride;
+  const __amdgpu_buffer_rsrc_t a_rsrc = make_rsrc(
+      p.a_src, static_cast<uint32_t>((PHASE == 1 ? p.tokens : 3 * p.tokens) * a_ld * 2));
+  auto source = [&](const Work& w) {
+    const uint16_t* base = w.t.seg == E ? p.w_shared
+                                        : p.w_routed + static_cast<int64_t>(w.t.seg) * w.N * w.K;
+    return make_rsrc(base, static_cast<uint32_t>(static_cast<int64_t>(w.N) * w.K * 2));
+  };
+  // Rows past the segment's end read some row (or zeros); they are not stored.
+  auto block_offsets = [&](const Work& w, int buf, uint32_t (&off)[6]) {
+    const int r0 = wave * 32 + (lane & 15);
+    int id[2];
+    if (PHASE == 1 && w.t.seg != E) {
+      asm volatile("ds_read_b32 %0, %2\n\tds_read_b32 %1, %2 offset:64\n\ts_waitcnt lgkmcnt(0)"
+                   : "=&v"(id[0]), "=&v"(id[1])
+                   : "v"(lds_addr(&ids_s[buf][r0])));
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int s = w.t.mt * kBigRows + r0 + 16 * i;
+      const int row = PHASE == 1 ? (w.t.seg == E ? s : id[i] >> 1) : w.t.hbase + s;
+      off[i] = (static_cast<uint32_t>(row) * a_ld + (lane >> 4) * 8) * 2u;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      off[2 + i] = static_cast<uint32_t>((w.n0 / 16 + wave * 4 + i) * (w.K / 32)) * 1024u + lane * 16u;
+  };
+
+  int at = static_cast<int>(blockIdx.x) >> 3;
+  if (at >= list_all) return;
+  Work cur = locate(at);
+  int parity = 0;
+  load_ids(cur, 0);
+  wait_vm_barrier<0>();
+  __amdgpu_buffer_rsrc_t src = source(cur);
+  uint32_t off[6];
+  block_offsets(cur, 0, off);
+  int ld_k = 0, slot_in = 0;  // next k step and ring slot to copy into
+  auto issue = [&]() {
+    const uint32_t ka = static_cast<uint32_t>(ld_k) * (kBigK * 2);
+    const uint32_t kb = static_cast<uint32_t>(ld_k) * 1024u;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      buffer_to_lds16(a_rsrc, &ring[slot_in][(wave * 2 + i) * 512], off[i], ka);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      buffer_to_lds16(src, &ring[slot_in][kBigRows * kBigK + (wave * 4 + i) * 512], off[2 + i], kb);
+    ++ld_k;
+    slot_in = slot_in == kBigStages - 1 ? 0 : slot_in + 1;
+  };
+#pragma unroll
+  for (int i = 0; i < kBigStages - 1; ++i) issue();
+
+  // Fragment addresses within a stage: token rows 32 i, packed weight rows
+  // 64 wave + 32 j (see grouped_gemm_wide_kernel for the layout).
+  const uint32_t lane_part = (lane >> 5) * 256u + (lane & 15) * 16u + ((lane & 31) >> 4) * 1024u;
+  const uint32_t ring0 = lds_addr(&ring[0][0]);
+  const uint32_t t_off = ring0 + lane_part;
+  const uint32_t w_off = ring0 + kBigRows * kBigK * 2 + wave * 4096u + lane_part;
+  int slot = 0;
+  bool follows = false;  // a tile's stores may precede this tile's k loop
+  bf16x8 a0[4], b0[2], a1[4], b1[2];  // a stage's two 16-wide k steps
+  auto products = [&](f32x16 (&acc)[2][4], const bf16x8 (&a)[4], const bf16x8 (&b)[2]) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[j], a[i], acc[j][i], 0, 0, 0);
+  };
+
+  for (;;) {
+    const int KT = cur.K / kBigK;
+    const bool has_next = at + step < list_all;
+    const Work next = locate(has_next ? at + step : at);
+    f32x16 acc[2][4];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[j][i][e] = 0.0f;
+
+    for (int kt = 0; kt < KT; ++kt) {
+      // Stage kt has landed for everybody, and everybody has read stage kt - 1.
+      if (follows && kt < kBigStages - 1) copies_left<kCopies + kStores>();
+      else copies_left<kCopies>();
+      join();
+      const uint32_t ta = t_off + slot * (kStageElems * 2u), wa = w_off + slot * (kStageElems * 2u);
+      slot = slot == kBigStages - 1 ? 0 : slot + 1;
+      if (kt == KT - (kBigStages - 1)) {
+        // from here on the copies are the next tile's (its row ids landed long ago)
+        src = source(next);
+        block_offsets(next, parity ^ 1, off);
+        ld_k = 0;
+      }
+      read_step6<0>(ta, wa, a0, b0);
+      // (everybody has left the epilogue that reads what these replace)
+      if (kt == 1) load_ids(next, parity ^ 1);
+      if (PHASE == 2 && kt == 2 && cur.t.seg != E && wave < kBigRows / kWave &&
+          cur.t.mt * kBigRows + tid < cur.t.rows) {
+        int id;
+        asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)"
+                     : "=&v"(id) : "v"(lds_addr(&ids_s[parity][tid])));
+        buffer_to_lds4(make_rsrc(p.weights, static_cast<uint32_t>(T) * 8u), &w_s[wave * kWave],
+                       static_cast<uint32_t>(id) * 4u);
+      }
+      products(acc, a0, b0);
+      issue();  // into the buffer of stage kt - 1
+      read_step6<512>(ta, wa, a1, b1);
+      products(acc, a1, b1);
+    }
+
+    // ---- epilogue: lane l holds token row l % 32 of each 32-row tile and
+    // packed weight rows 8 (e / 4) + 4 (l / 32) + e % 4 of each 32-row tile.
+    const bool shared = cur.t.seg == E;
+    // The stage just read is free until the next tile's first copies, which
+    // are issued after that tile's first barrier.
+    join();
+    const uint32_t out_lds =
+        ring0 + (slot == 0 ? kBigStages - 1 : slot - 1) * (kStageElems * 2u) + wave * (32 * kOutLd * 2u);
+    const int n = cur.n0 + wave * 64;  // this wavefront's first packed row
+    const int s0 = cur.t.mt * kBigRows + (lane >> 2);  // stored rows s0 + 16 m
+    constexpr uint32_t kNowhere = 0xfffffff0u;  // past any buffer: the store is dropped
+    if (PHASE == 1) {
+      const __amdgpu_buffer_rsrc_t out = make_rsrc(
+          p.hidden_out, static_cast<uint32_t>(static_cast<int64_t>(3) * T * p.hstride * 2));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        u32x2 v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {  // hidden values 8 q .. + 7 of the wavefront's 32
+          const int j = q >> 1, e = 4 * (q & 1);
+          float h[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) h[r] = swiglu(acc[j][i][e + r], acc[j][i][8 + e + r]);
+          v[q].x = pack_bf16x2(h[0], h[1]);
+          v[q].y = pack_bf16x2(h[2], h[3]);
+        }
+        u32x4 o[2];
+        rows_through_lds(out_lds, v, o);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const int s = s0 + 32 * i + 16 * k;
+          const uint32_t at_b =
+              (static_cast<uint32_t>(cur.t.hbase + s) * p.hstride + n / 2 + (lane & 3) * 8) * 2u;
+          __builtin_amdgcn_raw_buffer_store_b128(
+              o[k], out, s < cur.t.rows && n < cur.N ? at_b : kNowhere, 0, 0);
+        }
+      }
+    } else {
+      int id[8], wt[4];
+      read_dwords8(lds_addr(&ids_s[parity][lane >> 2]), id);
+      read_dwords4(lds_addr(&w_s[lane & 31]), wt);
+      const __amdgpu_buffer_rsrc_t out =
+          make_rsrc(shared ? p.y_shared : p.y_routed,
+                    static_cast<uint32_t>(static_cast<int64_t>(shared ? 1 : 2) * T * p.dim * 2));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float w = __int_as_float(wt[i]);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          u32x2 v[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            float y[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              y[r] = shared ? acc[j][i][4 * q + r] : w * acc[j][i][4 * q + r];
+            v[q].x = pack_bf16x2(y[0], y[1]);
+            v[q].y = pack_bf16x2(y[2], y[3]);
+          }
+          u32x4 o[2];
+          rows_through_lds(out_lds, v, o);
+#pragma unroll
+          for (int k = 0; k < 2; ++k) {
+            const int s = s0 + 32 * i + 16 * k;
+            const uint32_t row = static_cast<uint32_t>(shared ? s : id[2 * i + k]) * p.dim;
+            __builtin_amdgcn_raw_buffer_store_b128(
+                o[k], out,
+                s < cur.t.rows && n + 32 * j < cur.N ? (row + n + 32 * j + (lane & 3) * 8) * 2u : kNowhere, 0,
+                0);
+          }
+        }
+      }
+    }
+    if (!has_next) break;
+    at += step;
+    cur = next;
+    parity ^= 1;
+    follows = true;
+  }
+  // The copies issued past the last tile land before the LDS is given back.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
 // ---------------------------------------------------------------------------
@@ -1211,18 +1602,33 @@ hipError_t launch_phase(int phase, const GemmArgs& args, int n_max, hipStream_t 
   return hipGetLastError();
 }
 
-template <int BM, int BN, int BK, int S, int WAVES_M = 2, int WAVES_N = 2>
+template <int BM, int BN, int BK, int S>
 hipError_t launch_wide(int phase, const GemmArgs& args, int n_max, hipStream_t s) {
   const int T = static_cast<int>(args.tokens);
   const int m_tiles = (T + BM - 1) / BM + (2 * T) / BM + args.experts;
   // Rows of tiles rounded up to a multiple of the 8 XCDs (the kernel's tile
   // order takes every eighth row tile per XCD).
   const dim3 grid((n_max + BN - 1) / BN, (m_tiles + 7) / 8 * 8);
-  constexpr int kThreads = 64 * WAVES_M * WAVES_N;
-  if (phase == 1)
-    grouped_gemm_wide_kernel<BM, BN, BK, S, 1, WAVES_M, WAVES_N><<<grid, kThreads, 0, s>>>(args);
-  else
-    grouped_gemm_wide_kernel<BM, BN, BK, S, 2, WAVES_M, WAVES_N><<<grid, kThreads, 0, s>>>(args);
+  if (phase == 1) grouped_gemm_wide_kernel<BM, BN, BK, S, 1><<<grid, 256, 0, s>>>(args);
+  else grouped_gemm_wide_kernel<BM, BN, BK, S, 2><<<grid, 256, 0, s>>>(args);
+  return hipGetLastError();
+}
+
+// Whether the persistent kernel takes a wide launch: long enough k loops and
+// buffers that 32-bit offsets reach.
+bool persistent_applies(int phase, const GemmArgs& a) {
+  constexpr int64_t kReach = 0xfffffff0;  // the kernel's offset for dropped stores
+  const int k_min = phase == 1 ? a.dim : min(a.hidden_dim, a.shared_dim);
+  return k_min >= kBigKMin && int64_t{6} * a.tokens * a.hstride < kReach &&
+         int64_t{4} * a.tokens * a.dim < kReach &&
+         int64_t{4} * a.experts * a.capacity < kReach &&
+         int64_t{4} * a.dim * a.hstride < kReach;
+}
+
+hipError_t launch_persistent(int phase, const GemmArgs& args, hipStream_t s) {
+  constexpr int kGroups = 2 * 256;  // two per CU, a multiple of the 8 XCDs
+  if (phase == 1) grouped_gemm_big_kernel<1><<<kGroups, 256, 0, s>>>(args);
+  else grouped_gemm_big_kernel<2><<<kGroups, 256, 0, s>>>(args);
   return hipGetLastError();
 }
 
@@ -1269,24 +1675,19 @@ hipError_t run_stream(int phase, GemmArgs args, int n_max, hipStream_t s) {
 // K fits its LDS budget (64-row tiles in two k chunks, when every K splits
 // into 128-element halves; else 32-row tiles), else the pipelined kernel
 // with 32-row tiles.
-enum class TilePlan { kStream16, kStream32, kStream64, kWide128, kWide256 };
+enum class TilePlan { kStream16, kStream32, kStream64, kWide };
 
 // Average rows per expert from which the wide-MFMA tiles take over, per
-// phase.  Measured on MI355X (E = 16 uniform, T = 4K ... 64K, and BASELINE
-// config 3, E = 32 with 2 experts holding ~95 % of the rows): down is 18-31 %
-// faster on wide tiles from 256 rows per expert; gate/up only from 512 --
-// at config 3 its 30 small experts (~10 rows each) pay for whole 128 x 128
-// tiles with 1 KB x 24 weight blocks each (wide 49.8 us vs streaming 41.2).
+// phase.  They run on the persistent kernel, or where persistent_applies says
+// no on 128 x 128 tiles.  Measured on MI355X, streaming / persistent: down at
+// 256 rows per expert (T = 2048, E = 16) 18.4 / 17.3 us, (T = 4096, E = 32)
+// 28.6 / 22.8, and with two of the 32 experts holding ~95 % of the rows
+// 30.6 / 24.4.  Gate/up there 23.0 / 22.1, 40.8 / 33.9 and 31.8 / 31.0 us, but
+// streaming tiles group the rows themselves and the others need the grouping
+// launches first (7-10 us), so gate/up changes over at 512: T = 2048, E = 8
+// 26.9 -> 21.5 us; T = 4096, E = 16 37.9 -> 30.8 us.
 constexpr int64_t kWideRowsGateUp = 512;
 constexpr int64_t kWideRowsDown = 256;
-// Down on 256 x 256 tiles (eight wavefronts, one workgroup per CU) from this
-// many rows per expert.  Measured on MI355X (E = 16, HIP events): down
-// T = 32768 171 -> 163 us, T = 65536 327 -> 305 us; T = 16384 (2048 rows per
-// expert) 75 -> 82 us.  Gate/up stays on 128 x 128 tiles: 256 x 256 measured
-// 107 -> 156 us at T = 16384 and 385 -> 498 us at T = 65536 (with one
-// workgroup per CU nothing overlaps a tile's prologue and its hidden-tile
-// epilogue).
-constexpr int64_t kWide256RowsDown = 4096;
 
 template <TilePlan PLAN>
 hipError_t run_phase(int phase, GemmArgs args, const ExpertWeights& w, uint16_t* hidden,
@@ -1303,9 +1704,10 @@ hipError_t run_phase(int phase, GemmArgs args, const ExpertWeights& w, uint16_t*
     args.w_shared = w.shared_down;
     n_max = args.dim;
   }
-  if constexpr (PLAN == TilePlan::kWide128) return launch_wide<128, 128, 32, 3>(phase, args, n_max, s);
-  if constexpr (PLAN == TilePlan::kWide256)
-    return launch_wide<256, 256, 32, 4, 2, 4>(phase, args, n_max, s);
+  if constexpr (PLAN == TilePlan::kWide) {
+    if (persistent_applies(phase, args)) return launch_persistent(phase, args, s);
+    return launch_wide<128, 128, 32, 3>(phase, args, n_max, s);
+  }
   const int k_max = phase == 1 ? args.dim : max(args.hidden_dim, args.shared_dim);
   if (k_max > kStreamKCap) return launch_phase<32, 128, 3>(phase, args, n_max, s);
   if constexpr (PLAN == TilePlan::kStream64) {
@@ -1325,14 +1727,13 @@ hipError_t run_phase(int phase, GemmArgs args, const ExpertWeights& w, uint16_t*
 // expert the weight fragments' trips from L2 set the pace (each 32-row tile
 // of an expert re-reads its weights), and 64-row tiles in two k chunks halve
 // them.  From kWideRowsGateUp / kWideRowsDown rows per expert the wide-MFMA
-// 128 x 128 tiles take over (grouped_gemm_wide_kernel).
+// tiles take over (grouped_gemm_big_kernel).
 TilePlan experts_tile_plan(int phase, int64_t tokens, int experts) {
   const int64_t per_expert = (2 * tokens + experts - 1) / experts;
   if (tokens <= 16) return TilePlan::kStream16;
   if (per_expert <= 96) return TilePlan::kStream32;
   const int64_t wide_from = phase == 1 ? kWideRowsGateUp : kWideRowsDown;
-  if (per_expert < wide_from) return TilePlan::kStream64;
-  return phase == 2 && per_expert >= kWide256RowsDown ? TilePlan::kWide256 : TilePlan::kWide128;
+  return per_expert < wide_from ? TilePlan::kStream64 : TilePlan::kWide;
 }
 
 // Streaming-kernel tile order for gate/up: row-major per XCD once the
@@ -1356,7 +1757,7 @@ GroupInKernel experts_group_in_kernel(int64_t tokens, int dim, int experts, int 
   if (tokens < 1 || experts > kMaxExperts) return kGroupNone;
   if (dim > kStreamKCap || max(hidden_dim, shared_dim) > kStreamKCap) return kGroupNone;
   // The streaming kernel groups; the wide tiles' plan does not.
-  if (experts_tile_plan(1, tokens, experts) == TilePlan::kWide128) return kGroupNone;
+  if (experts_tile_plan(1, tokens, experts) == TilePlan::kWide) return kGroupNone;
   // From the ids: up to ~3 x 32 rows per expert on average (the shapes it
   // was measured at).
   if (2 * tokens <= kGroupMaxAssign && (2 * tokens + experts - 1) / experts <= 96)
@@ -1404,8 +1805,7 @@ hipError_t launch_expert_gemm(int phase, const uint16_t* x, int64_t tokens, int 
     case TilePlan::kStream16: return run_phase<TilePlan::kStream16>(phase, args, w, hidden, s);
     case TilePlan::kStream32: return run_phase<TilePlan::kStream32>(phase, args, w, hidden, s);
     case TilePlan::kStream64: return run_phase<TilePlan::kStream64>(phase, args, w, hidden, s);
-    case TilePlan::kWide128: return run_phase<TilePlan::kWide128>(phase, args, w, hidden, s);
-    default: return run_phase<TilePlan::kWide256>(phase, args, w, hidden, s);
+    default: return run_phase<TilePlan::kWide>(phase, args, w, hidden, s);
   }
 }
 
