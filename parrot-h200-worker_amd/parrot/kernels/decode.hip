@@ -468,8 +468,9 @@ __global__ __launch_bounds__(256) void decode_split_kernel(
     const int h = wave + 4 * i;
     const float v = s_s[h][lane];
     const float m = wave_max(v);
-    // A chunk whose scores are all -inf weighs nothing.
-    const float e = m == -INFINITY ? 0.0f : __expf(v - m);
+    // A chunk whose scores are all -inf weighs nothing; the maximum passes
+    // over NaN scores, which stay NaN.
+    const float e = m == -INFINITY && v == v ? 0.0f : __expf(v - m);
     const float l = wave_sum(e);
     s_s[h][lane] = e;  // read back by this wavefront only
     if (lane == 0 && h < rep)

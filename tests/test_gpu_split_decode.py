@@ -72,6 +72,25 @@ def test_split_decode_attention(monkeypatch, b, H, Hk, d, max_pos, window, posit
     assert ((heads.double() - want).abs() <= 1e-6 * size + 1e-7).all()
 
 
+# the NaN key alone in the last chunk, beside others, and in a full first chunk
+@pytest.mark.parametrize("position,nan_key", [(64, 64), (70, 70), (130, 5), (255, 255)])
+def test_split_decode_attention_nan_key(monkeypatch, position, nan_key):
+    """A NaN in a key reaches the outputs of the heads that read it, wherever
+    the key falls among the chunks, as in the one-launch form."""
+    hip_moe = _split_always(monkeypatch)
+    print(f"split decode NaN key {nan_key} p={position}", flush=True)
+    q, kn, vn, kc, vc = _local_inputs(1, 8, 2, 96, 256, position)
+    (kn[:, 0, 0] if nan_key == position else kc[:, 0, nan_key])[:, 3] = float("nan")
+    pos = torch.tensor([position], dtype=torch.int32, device="cuda")
+    with torch.no_grad():
+        one, got = (hip_moe.decode_attention(q, kn, vn, kc.clone(), vc.clone(), pos, 256,
+                                             96 ** -0.5, context=context)
+                    for context in (None, position + 1))
+    for out in (one, got):
+        rows = out.view(8, 96)
+        assert rows[:4].isnan().all() and not rows[4:].isnan().any()
+
+
 @pytest.mark.parametrize("b,H,r,position", [(1, 8, 128, 0), (2, 8, 128, 64), (3, 6, 128, 700),
                                             (1, 16, 64, 129), (2, 3, 32, 383)])
 def test_split_decode_attention_latent(monkeypatch, b, H, r, position):
