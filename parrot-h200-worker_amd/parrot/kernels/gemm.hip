@@ -951,53 +951,73 @@ void grouped_gemm_wide_kernel(GemmArgs p) {
 // (or 16) k steps of a tile; and with two independent workgroups on a CU one
 // multiplies while the other waits, applies SwiGLU or stores.
 //
-//   stages    32 k values of A (128 gathered rows) and B (256 packed weight
-//             rows), 24 KB, direct to LDS in a ring of three.
+//   rows      32 k values of 128 gathered rows, 8 KB a stage, direct to LDS in
+//             a ring of three.
+//   weights   no two wavefronts of a workgroup need the same ones, so each
+//             streams the fragments of its own 64 packed rows from L2 into
+//             registers, two k steps ahead: 20 KB of LDS traffic per 16 k
+//             values instead of 36 KB with the weights through LDS too.
 //   products  v_mfma_f32_32x32x16_bf16 with the weights as the A operand: a
 //             lane then holds one token row of each 32-row tile and, of every
 //             32 packed gate / up rows, 8 gate values and their 8 up values,
 //             so SwiGLU needs no exchange and a lane needs one route weight per
-//             32-row tile.  Rows leave through the stage buffer just read, as
+//             32-row tile.  Rows leave through the wavefront's own LDS rows, as
 //             64-byte runs.
 //   row ids   direct to LDS too (one dword copy per row), so nothing in the
-//             loop waits for a register load.
+//             loop waits for a register load of them.
+//   order     an XCD takes consecutive routed row tiles, so that its workgroups
+//             share the weights of one or two experts in its L2; dealt out in
+//             turn (row tile % 8) each of the eight L2s pulled in every expert
+//             and a round's 64 tiles spanned four: 3.9 million L2 misses of 128
+//             bytes per gate/up launch at 32768 tokens against 2.5 million.
 //
-// Waits: every wavefront issues kCopies copies per stage; stage kt has landed
-// when at most those of stage kt + 1 are outstanding.  Stages 0 and 1 of a
-// tile were issued before the previous tile's kStores stores, which may be
+// Waits: every wavefront issues kLoads copies and loads per k step; stage kt has
+// landed when at most those of step kt - 1 are outstanding.  Stages 0 and 1 of
+// a tile were issued before the previous tile's kStores stores, which may be
 // outstanding as well (vector-memory operations retire in order).  Row id and
 // route weight copies only make those waits stricter.  A tile needs 7 k steps
 // for its successor's row ids and its own route weights to land in time
 // (kBigKMin asks for 8).
 //
-// Bound by the matrix cores together with what the wavefronts issue beside
-// them: with 256 x 256 tiles, of gate/up's 157 us at 32768 tokens, leaving out
-// the products, the copies or the LDS reads saved 15-20 us each, the epilogue
-// 35.  Measured on MI355X at 32768 tokens, 16 experts (a graph of 10
-// launches, 128 x 128 tiles of one workgroup each / this): gate/up 211 /
-// 147 us (1.05 PFLOP/s), down 133 / 89 us.  65536 tokens: 373 / 281 and
-// 276 / 204.  16384: 119 / 85 and 76 / 49.  256 x 256 tiles in one workgroup of
-// eight wavefronts per CU, in step or half a stage apart: 157-166 and 92-97.
-// Copies issued after a stage's first products instead of before: 168 -> 162.
+// Bound by what feeds the matrix cores: with the weights through LDS and the
+// row tiles dealt out in turn they were busy 41 % of gate/up's cycles (at 2.06
+// GHz under this load) while 15 TB/s came out of the L2s.  Neither
+// half measure helps alone: with the row tiles dealt out in turn, weights in
+// registers left the MoE layer of 32768 tokens as it was (two or four k steps
+// ahead); consecutive row tiles with the weights through LDS took it from 329
+// to 324 us, both together to 313.  Four k steps ahead and a ring of five, then,
+// 316 us; raised wave priority around the products 319 us.
+//
+// Measured on MI355X at 32768 tokens, 16 experts (a graph of 10 launches, one
+// workgroup per 128 x 128 tile / persistent, weights through LDS and tiles in
+// turn): gate/up 211 / 147 us, down 133 / 89 us; 65536 tokens 373 / 281 and
+// 276 / 204; 16384 tokens 119 / 85 and 76 / 49.  The form here against that one
+// (kernel trace of the eager layer, 32768 tokens): gate/up 156 -> 139 us
+// (0.93 PFLOP/s), down 103 -> 98 us; 4096 skewed tokens, 32 experts, down
+// 23.3 -> 22.0 us.
+//
+// 256 x 256 tiles in one workgroup of eight wavefronts per CU (weights through
+// LDS), in step or half a stage apart: gate/up 157-166 and down 92-97 us where
+// 128 x 256 tiles took 147 and 89.  Copies issued after a stage's first
+// products instead of before: 168 -> 162 there.
 constexpr int kBigRows = 128;
 constexpr int kBigCols = 256;
 constexpr int kBigK = 32;       // k values per stage
-constexpr int kBigStages = 3;
+constexpr int kBigAhead = 2;    // k steps in flight; K is a multiple of 2 kBigK
+constexpr int kBigStages = kBigAhead + 1;
 constexpr int kBigKMin = 8 * kBigK;
 
-// One 16-wide k step's six fragments from LDS, landed on return: token rows at
-// `t` + 2048 i + O, weight rows at `w` + 2048 j + O (one asm block: no register
-// is named before its data is there, and the compiler ties nothing to the
-// copies in flight).
+// One 16-wide k step's fragments of the token rows from LDS, landed on return:
+// rows 32 i at `t` + 2048 i + O (one asm block: no register is named before its
+// data is there, and the compiler ties nothing to the copies in flight).
 template <int O>
-__device__ __forceinline__ void read_step6(uint32_t t, uint32_t w, bf16x8 (&a)[4], bf16x8 (&b)[2]) {
+__device__ __forceinline__ void read_rows4(uint32_t t, bf16x8 (&a)[4]) {
   asm volatile(
-      "ds_read_b128 %4, %7 offset:%8\n\tds_read_b128 %0, %6 offset:%8\n\t"
-      "ds_read_b128 %5, %7 offset:%9\n\tds_read_b128 %1, %6 offset:%9\n\t"
-      "ds_read_b128 %2, %6 offset:%10\n\tds_read_b128 %3, %6 offset:%11\n\t"
+      "ds_read_b128 %0, %4 offset:%5\n\tds_read_b128 %1, %4 offset:%6\n\t"
+      "ds_read_b128 %2, %4 offset:%7\n\tds_read_b128 %3, %4 offset:%8\n\t"
       "s_waitcnt lgkmcnt(0)"
-      : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2]), "=&v"(a[3]), "=&v"(b[0]), "=&v"(b[1])
-      : "v"(t), "v"(w), "i"(O), "i"(O + 2048), "i"(O + 4096), "i"(O + 6144));
+      : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2]), "=&v"(a[3])
+      : "v"(t), "i"(O), "i"(O + 2048), "i"(O + 4096), "i"(O + 6144));
 }
 
 __device__ __forceinline__ void join() { asm volatile("s_barrier" ::: "memory"); }
@@ -1060,10 +1080,11 @@ __device__ __forceinline__ void buffer_to_lds4(__amdgpu_buffer_rsrc_t r, void* l
 
 template <int PHASE>
 __global__ __launch_bounds__(256, 2) void grouped_gemm_big_kernel(GemmArgs p) {
-  constexpr int kStageElems = (kBigRows + kBigCols) * kBigK;
-  constexpr int kCopies = 6;  // per wavefront and stage
+  constexpr int kStageElems = kBigRows * kBigK;
+  constexpr int kLoads = 6;  // per wavefront and k step: two copies, four weight fragments
   constexpr int kStores = PHASE == 1 ? 8 : 16;  // per wavefront and tile, always issued
   __shared__ __attribute__((aligned(16))) uint16_t ring[kBigStages][kStageElems];
+  __shared__ __attribute__((aligned(16))) uint16_t out_s[4][32 * kOutLd];
   __shared__ int ids_s[2][kBigRows];   // assignment ids of the routed rows, by tile parity
   __shared__ int w_s[kBigRows];        // their route weights (phase 2)
 
@@ -1088,10 +1109,13 @@ __global__ __launch_bounds__(256, 2) void grouped_gemm_big_kernel(GemmArgs p) {
   const int Ns = PHASE == 1 ? 2 * p.shared_dim : p.dim;
   const int nr = (Nr + kBigCols - 1) / kBigCols, ns = (Ns + kBigCols - 1) / kBigCols;
 
-  // This XCD's tiles: row tiles x, x + 8, ... with all their column tiles in
-  // turn, the routed ones first; this workgroup takes every gridDim / 8-th.
+  // This XCD's tiles: an eighth of the routed row tiles, consecutive ones (of
+  // one or two experts at a time, whose weights then stay in its L2), with all
+  // their column tiles in turn, then shared row tiles x, x + 8, ...; this
+  // workgroup takes every gridDim / 8-th.
   const int xcd = static_cast<int>(blockIdx.x) & 7;
-  const int list_r = ((routed_m + 7 - xcd) >> 3) * nr;
+  const int first_m = xcd * routed_m / 8;
+  const int list_r = ((xcd + 1) * routed_m / 8 - first_m) * nr;
   const int list_all = list_r + ((shared_m + 7 - xcd) >> 3) * ns;
   const int step = static_cast<int>(gridDim.x) >> 3;
 
@@ -1103,7 +1127,7 @@ __global__ __launch_bounds__(256, 2) void grouped_gemm_big_kernel(GemmArgs p) {
     Work w;
     if (i < list_r) {
       const int q = i / nr;
-      const int m = xcd + 8 * q;
+      const int m = first_m + q;
       const uint64_t hit = __ballot(mine && m >= tile0 && m < tile_end);
       const int seg = static_cast<int>(__builtin_ctzll(hit));
       w.t = Tile{seg, m - __builtin_amdgcn_readlane(tile0, seg),
@@ -1142,8 +1166,9 @@ __global__ __launch_bounds__(256, 2) void grouped_gemm_big_kernel(GemmArgs p) {
     }
   };
 
-  // Copy state: each wavefront copies two of a stage's eight 1 KB blocks of A
-  // (16 rows x 32 k values) and four of its sixteen blocks of B.
+  // Load state: each wavefront copies two of a stage's eight 1 KB blocks of token
+  // rows (16 rows x 32 k values) and loads the four fragments of its own 64
+  // packed weight rows (32 rows x 16 k values each).
   const int a_ld = PHASE == 1 ? p.dim : p.hstride;
   const __amdgpu_buffer_rsrc_t a_rsrc = make_rsrc(
       p.a_src, static_cast<uint32_t>((PHASE == 1 ? p.tokens : 3 * p.tokens) * a_ld * 2));
@@ -1153,7 +1178,7 @@ __global__ __launch_bounds__(256, 2) void grouped_gemm_big_kernel(GemmArgs p) {
     return make_rsrc(base, static_cast<uint32_t>(static_cast<int64_t>(w.N) * w.K * 2));
   };
   // Rows past the segment's end read some row (or zeros); they are not stored.
-  auto block_offsets = [&](const Work& w, int buf, uint32_t (&off)[6]) {
+  auto block_offsets = [&](const Work& w, int buf, uint32_t (&off)[4]) {
     const int r0 = wave * 32 + (lane & 15);
     int id[2];
     if (PHASE == 1 && w.t.seg != E) {
@@ -1168,8 +1193,10 @@ __global__ __launch_bounds__(256, 2) void grouped_gemm_big_kernel(GemmArgs p) {
       off[i] = (static_cast<uint32_t>(row) * a_ld + (lane >> 4) * 8) * 2u;
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      off[2 + i] = static_cast<uint32_t>((w.n0 / 16 + wave * 4 + i) * (w.K / 32)) * 1024u + lane * 16u;
+    for (int j = 0; j < 2; ++j)
+      off[2 + j] = static_cast<uint32_t>((w.n0 / 16 + wave * 4 + 2 * j) * (w.K / 32) +
+                                         ((lane & 31) >> 4) * (w.K / 32)) * 1024u +
+                   (lane >> 5) * 256u + (lane & 15) * 16u;
   };
 
   int at = static_cast<int>(blockIdx.x) >> 3;
@@ -1179,39 +1206,44 @@ __global__ __launch_bounds__(256, 2) void grouped_gemm_big_kernel(GemmArgs p) {
   load_ids(cur, 0);
   wait_vm_barrier<0>();
   __amdgpu_buffer_rsrc_t src = source(cur);
-  uint32_t off[6];
+  uint32_t off[4];
   block_offsets(cur, 0, off);
-  int ld_k = 0, slot_in = 0;  // next k step and ring slot to copy into
-  auto issue = [&]() {
+  int ld_k = 0, slot_in = 0;  // next k step to load and ring slot to copy into
+  auto copy_rows = [&]() {
     const uint32_t ka = static_cast<uint32_t>(ld_k) * (kBigK * 2);
-    const uint32_t kb = static_cast<uint32_t>(ld_k) * 1024u;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
       buffer_to_lds16(a_rsrc, &ring[slot_in][(wave * 2 + i) * 512], off[i], ka);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      buffer_to_lds16(src, &ring[slot_in][kBigRows * kBigK + (wave * 4 + i) * 512], off[2 + i], kb);
-    ++ld_k;
     slot_in = slot_in == kBigStages - 1 ? 0 : slot_in + 1;
   };
+  // Half h (16 k values) of k step ld_k of the wavefront's weight rows.
+  auto load_weights = [&](uint4 (&b)[2], int h) {
 #pragma unroll
-  for (int i = 0; i < kBigStages - 1; ++i) issue();
+    for (int j = 0; j < 2; ++j)
+      b[j] = buffer_load16(src, off[2 + j] + h * 512u, static_cast<uint32_t>(ld_k) * 1024u);
+  };
+  uint4 bq[kBigAhead][2][2];  // [k step parity][half][32-row group]
+#pragma unroll
+  for (int i = 0; i < kBigAhead; ++i) {
+    copy_rows();
+    load_weights(bq[i][0], 0);
+    load_weights(bq[i][1], 1);
+    ++ld_k;
+  }
 
-  // Fragment addresses within a stage: token rows 32 i, packed weight rows
-  // 64 wave + 32 j (see grouped_gemm_wide_kernel for the layout).
-  const uint32_t lane_part = (lane >> 5) * 256u + (lane & 15) * 16u + ((lane & 31) >> 4) * 1024u;
-  const uint32_t ring0 = lds_addr(&ring[0][0]);
-  const uint32_t t_off = ring0 + lane_part;
-  const uint32_t w_off = ring0 + kBigRows * kBigK * 2 + wave * 4096u + lane_part;
+  // Fragment address within a stage: token rows 32 i (see
+  // grouped_gemm_wide_kernel for the layout).
+  const uint32_t t_off = lds_addr(&ring[0][0]) + (lane >> 5) * 256u + (lane & 15) * 16u +
+                         ((lane & 31) >> 4) * 1024u;
   int slot = 0;
   bool follows = false;  // a tile's stores may precede this tile's k loop
-  bf16x8 a0[4], b0[2], a1[4], b1[2];  // a stage's two 16-wide k steps
-  auto products = [&](f32x16 (&acc)[2][4], const bf16x8 (&a)[4], const bf16x8 (&b)[2]) {
+  auto products = [&](f32x16 (&acc)[2][4], const bf16x8 (&a)[4], const uint4 (&b)[2]) {
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[j], a[i], acc[j][i], 0, 0, 0);
+        acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, b[j]), a[i],
+                                                            acc[j][i], 0, 0, 0);
   };
 
   for (;;) {
@@ -1226,20 +1258,21 @@ __global__ __launch_bounds__(256, 2) void grouped_gemm_big_kernel(GemmArgs p) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[j][i][e] = 0.0f;
 
-    for (int kt = 0; kt < KT; ++kt) {
+    auto k_step = [&](int kt, uint4 (&b)[2][2]) {
       // Stage kt has landed for everybody, and everybody has read stage kt - 1.
-      if (follows && kt < kBigStages - 1) copies_left<kCopies + kStores>();
-      else copies_left<kCopies>();
+      if (follows && kt < kBigAhead) copies_left<kLoads + kStores>();
+      else copies_left<kLoads>();
       join();
-      const uint32_t ta = t_off + slot * (kStageElems * 2u), wa = w_off + slot * (kStageElems * 2u);
+      const uint32_t ta = t_off + slot * (kStageElems * 2u);
       slot = slot == kBigStages - 1 ? 0 : slot + 1;
-      if (kt == KT - (kBigStages - 1)) {
-        // from here on the copies are the next tile's (its row ids landed long ago)
+      if (kt == KT - kBigAhead) {
+        // from here on the loads are the next tile's (its row ids landed long ago)
         src = source(next);
         block_offsets(next, parity ^ 1, off);
         ld_k = 0;
       }
-      read_step6<0>(ta, wa, a0, b0);
+      bf16x8 a[4];
+      read_rows4<0>(ta, a);
       // (everybody has left the epilogue that reads what these replace)
       if (kt == 1) load_ids(next, parity ^ 1);
       if (PHASE == 2 && kt == 2 && cur.t.seg != E && wave < kBigRows / kWave &&
@@ -1250,20 +1283,27 @@ __global__ __launch_bounds__(256, 2) void grouped_gemm_big_kernel(GemmArgs p) {
         buffer_to_lds4(make_rsrc(p.weights, static_cast<uint32_t>(T) * 8u), &w_s[wave * kWave],
                        static_cast<uint32_t>(id) * 4u);
       }
-      products(acc, a0, b0);
-      issue();  // into the buffer of stage kt - 1
-      read_step6<512>(ta, wa, a1, b1);
-      products(acc, a1, b1);
+      products(acc, a, b[0]);
+      copy_rows();  // into the buffer of stage kt - 1
+      load_weights(b[0], 0);
+      __builtin_amdgcn_sched_barrier(0);
+      read_rows4<512>(ta, a);
+      products(acc, a, b[1]);
+      load_weights(b[1], 1);
+      __builtin_amdgcn_sched_barrier(0);
+      ++ld_k;
+    };
+#pragma unroll 1
+    for (int kt = 0; kt < KT; kt += kBigAhead) {
+      static_assert(kBigAhead == 2, "one call per k step in flight");
+      k_step(kt, bq[0]);
+      k_step(kt + 1, bq[1]);
     }
 
     // ---- epilogue: lane l holds token row l % 32 of each 32-row tile and
     // packed weight rows 8 (e / 4) + 4 (l / 32) + e % 4 of each 32-row tile.
     const bool shared = cur.t.seg == E;
-    // The stage just read is free until the next tile's first copies, which
-    // are issued after that tile's first barrier.
-    join();
-    const uint32_t out_lds =
-        ring0 + (slot == 0 ? kBigStages - 1 : slot - 1) * (kStageElems * 2u) + wave * (32 * kOutLd * 2u);
+    const uint32_t out_lds = lds_addr(&out_s[wave][0]);
     const int n = cur.n0 + wave * 64;  // this wavefront's first packed row
     const int s0 = cur.t.mt * kBigRows + (lane >> 2);  // stored rows s0 + 16 m
     constexpr uint32_t kNowhere = 0xfffffff0u;  // past any buffer: the store is dropped
