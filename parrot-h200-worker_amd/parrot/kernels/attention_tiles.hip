@@ -39,6 +39,7 @@
 // 1 x 2047 37 / 40 / 26; 2 x 512 11.4 / 13.9 / 10.2; 3 x 333 9.4 / 10.5 /
 // 8.8; 1 x 1000 14.5 / 21.4 / 15.3; 1 x 512 6.7 / 13.3 / 10.0.
 #include "common.h"
+#include "extents.h"
 
 namespace parrot {
 
@@ -138,7 +139,7 @@ __global__ __launch_bounds__(256, 2) void attention_tile_kernel(TileArgs a) {
   constexpr int kStageElems = 2 * SB * kBlockElems;  // the K blocks, then the V blocks
   constexpr int kPieces = kStageElems / 512;       // 1 KB copies per stage
   constexpr int kCopies = kPieces / 4;             // per wavefront
-  constexpr int NB = 2;                            // ring of stages in LDS
+  constexpr int NB = 2;                            // stages in LDS, used in turn
   static_assert(kCopies * 4 == kPieces, "whole copies per wavefront");
   static_assert(KG == 1 || KG == 2, "key groups");
   __shared__ __attribute__((aligned(16))) uint16_t stage[NB][kStageElems];
@@ -177,20 +178,21 @@ __global__ __launch_bounds__(256, 2) void attention_tile_kernel(TileArgs a) {
   const __amdgpu_buffer_rsrc_t v_rsrc =
       make_rsrc(a.vf + static_cast<int64_t>(bh) * nblk * kBlockElems,
                 static_cast<uint32_t>(nblk) * kBlockElems * 2);
-  // One stage: SB key blocks of K then of V, 1 KB per wavefront copy (blocks
-  // past the sequence read as zero).
+  // One stage: SB key blocks of K then of V, 1 KB per wavefront copy.  The
+  // second block of an odd last pair is the first once more (no query sees it):
+  // the scalar offset that says which block is read lies inside the buffer.
   auto issue = [&](int st, int buf) {
-    const uint32_t base = static_cast<uint32_t>(lo + st * SB) * (kBlockElems * 2);
+    const int first = lo + st * SB;
 #pragma unroll
     for (int i = 0; i < kCopies; ++i) {
       const int piece = i * 4 + wave;
       const bool is_v = piece >= kPieces / 2;
-      const uint32_t off = static_cast<uint32_t>(is_v ? piece - kPieces / 2 : piece) * 1024u;
-      buffer_to_lds16(is_v ? v_rsrc : k_rsrc, &stage[buf][piece * 512], lane * 16u, base + off);
+      buffer_to_lds16(is_v ? v_rsrc : k_rsrc, &stage[buf][piece * 512], lane * 16u,
+                      stage_piece_offset(first, is_v ? piece - kPieces / 2 : piece,
+                                         kPieces / (2 * SB), nblk));
     }
   };
-#pragma unroll
-  for (int i = 0; i < NB - 1; ++i) issue(i, i);
+  issue(0, 0);
 
   // Q^T as the B operand: lane holds query q0 + col, dims 16 u + 8 half .. + 7.
   bf16x8 qf[KU];
@@ -317,11 +319,11 @@ __global__ __launch_bounds__(256, 2) void attention_tile_kernel(TileArgs a) {
       reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const uint16_t*)&stage[0][0]));
   int buf = 0;
   for (int st = 0; st < stages; ++st) {
-    // This wavefront's copies of stage st have landed (those of NB - 2 later
-    // stages may be in flight); past the barrier everybody's have, and nobody
-    // reads the buffer of stage st - 1 any more.
-    wait_vm_barrier<(NB - 2) * kCopies>();
-    issue(st + NB - 1, buf == 0 ? NB - 1 : buf - 1);
+    // This wavefront's copies of stage st, the only ones in flight, have
+    // landed; past the barrier everybody's have, and nobody reads the buffer
+    // of stage st - 1 any more.
+    wait_vm_barrier<0>();
+    if (st + 1 < stages) issue(st + 1, buf ^ 1);
     // Blocks past this wavefront's diagonal or before its window are left out.
     const uint32_t lds = lds0 + buf * (kStageElems * 2);
     const int k0 = (lo + st * SB) * 32;
@@ -329,12 +331,9 @@ __global__ __launch_bounds__(256, 2) void attention_tile_kernel(TileArgs a) {
 #pragma unroll
     for (int j = kw; j < SB; j += KG)
       if (seen(k0 + 32 * j)) block(lds + j * kNext, k0 + 32 * j);
-    buf = buf + 1 == NB ? 0 : buf + 1;
+    buf ^= 1;
   }
   l += __shfl_xor(l, 32);
-  // The copies still in flight land before the buffers are used again or
-  // given back.
-  wait_vm_barrier<0>();
 
   // The other key groups hand their states to group 0 through the stage
   // buffers; it adds them in group order.
@@ -342,6 +341,7 @@ __global__ __launch_bounds__(256, 2) void attention_tile_kernel(TileArgs a) {
     constexpr int kState = DT * 16 * kWave;  // floats per wavefront
     static_assert((4 - 4 / KG) * kState * 4 <= NB * kStageElems * 2, "the merge fits the stages");
     float* ob = reinterpret_cast<float*>(&stage[0][0]);
+    __syncthreads();  // everybody has read the last stage
     if (kw > 0) {
       const int at = slot * (KG - 1) + kw - 1;
 #pragma unroll

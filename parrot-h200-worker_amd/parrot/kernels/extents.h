@@ -1,0 +1,28 @@
+// How far the tiled kernels' copies and loads reach, as plain functions of the
+// sizes: the kernels take their offsets from them, and a host program can walk
+// a whole launch through them.
+//
+// A buffer descriptor's bound covers the per-lane offset.  Whether it covers
+// the scalar offset too is not something to rely on, so a scalar offset always
+// names a place inside the buffer.
+#pragma once
+
+#include <cstdint>
+
+#ifdef __HIP__
+#define PARROT_EXTENT __host__ __device__ __forceinline__ constexpr
+#else
+#define PARROT_EXTENT inline constexpr
+#endif
+
+namespace parrot {
+
+// attention_tiles.hip: byte offset in one kv head's K (or V) fragments, nblk
+// blocks of `pieces` KB, of KB `piece` of the two blocks from `first` on.
+PARROT_EXTENT uint32_t stage_piece_offset(int first, int piece, int pieces, int nblk) {
+  const bool second = piece >= pieces;
+  const int block = second && first + 1 < nblk ? first + 1 : first;
+  return static_cast<uint32_t>(block * pieces + (second ? piece - pieces : piece)) * 1024u;
+}
+
+}  // namespace parrot

@@ -1,0 +1,45 @@
+"""Every offset that the tiled kernels' copies and loads take lies inside the
+buffer it is taken in: the kernels' own index functions, compiled for the host
+and walked through whole launches."""
+import subprocess
+from pathlib import Path
+
+KERNELS = Path(__file__).resolve().parent.parent / "parrot-h200-worker_amd" / "parrot" / "kernels"
+
+
+def _run(tmp_path, body):
+    source, program = tmp_path / "walk.cpp", tmp_path / "walk"
+    source.write_text('#include "extents.h"\n#include <algorithm>\n#include <cstdio>\n'
+                      "using namespace parrot;\nint main() {\n" + body + "\n}\n")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", f"-I{KERNELS}", str(source), "-o",
+                    str(program)], check=True)
+    done = subprocess.run([str(program)], capture_output=True, text=True)
+    assert done.returncode == 0, done.stdout
+
+
+def test_attention_stages_stay_inside_the_fragments(tmp_path):
+    """Every sequence length over several blocks, windows inside a block and
+    longer than the sequence, every query tile, both blocks of each stage."""
+    _run(tmp_path, """
+  for (int d : {64, 96, 128})
+    for (int T = 1; T <= 330; ++T)
+      for (int W : {1, 33, 77, 4096})
+        for (int rows : {32, 64, 128})  // queries per workgroup
+          for (int wg0 = 0; wg0 < T; wg0 += rows) {
+            const int nblk = (T + 31) / 32, pieces = d / 16;
+            const long bytes = static_cast<long>(nblk) * 32 * d * 2;
+            const int lo = std::max(0, wg0 - W + 1) / 32;
+            const int stages = ((std::min(wg0 + rows, T) - 1) / 32 - lo) / 2 + 1;
+            for (int st = 0; st < stages; ++st)
+              for (int piece = 0; piece < 2 * pieces; ++piece) {
+                const long at = stage_piece_offset(lo + 2 * st, piece, pieces, nblk);
+                const int block = lo + 2 * st + piece / pieces;
+                const long want = (static_cast<long>(std::min(block, nblk - 1)) * pieces + piece % pieces) * 1024;
+                if (at + 1024 > bytes || at != want) {
+                  std::printf("d=%d T=%d W=%d wg0=%d stage %d piece %d: %ld of %ld\\n", d, T, W, wg0,
+                              st, piece, at, bytes);
+                  return 1;
+                }
+              }
+          }
+  return 0;""")
