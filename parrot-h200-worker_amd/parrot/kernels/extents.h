@@ -25,4 +25,12 @@ PARROT_EXTENT uint32_t stage_piece_offset(int first, int piece, int pieces, int 
   return static_cast<uint32_t>(block * pieces + (second ? piece - pieces : piece)) * 1024u;
 }
 
+// proj.hip, many rows: byte offset in the packed weight (N columns, ksteps
+// 32-wide k steps) of k step `step` of the 16-column group `group` of the block
+// that starts at column col0.
+PARROT_EXTENT uint32_t column_group_offset(int col0, int group, int N, int ksteps, int step) {
+  const int at = col0 / 16 + group, last = N / 16 - 1;
+  return static_cast<uint32_t>((at < last ? at : last) * ksteps + step) * 1024u;
+}
+
 }  // namespace parrot

@@ -44,6 +44,7 @@
 //             grouped into heads of head_dim, or both from one [Wk; Wv]
 //             weight (the MLA up-projections).
 #include "common.h"
+#include "extents.h"
 
 #include <type_traits>
 
@@ -528,12 +529,14 @@ __global__ __launch_bounds__(64 * NW, 2) void proj_rows_kernel(ProjArgs p, int s
   const __amdgpu_buffer_rsrc_t b_rsrc =
       make_rsrc(p.w, static_cast<uint32_t>(static_cast<int64_t>(p.N) * K * 2));
   uint4 bq[PF][kBlockGroups];
-  // Step `step` of the block whose first column is col0 (columns past N read 0).
+  // Step `step` of the block whose first column is col0 (groups past the last
+  // one read it: the scalar offset stays inside the weights, and what comes of
+  // them is not stored).
   auto load_step = [&](uint4 (&dst)[kBlockGroups], int col0, int step) {
 #pragma unroll
     for (int j = 0; j < kBlockGroups; ++j)
       dst[j] = buffer_load16(b_rsrc, lane * 16u,
-                             static_cast<uint32_t>((col0 / 16 + j) * KST + step) * 1024u);
+                             column_group_offset(col0, j, p.N, KST, step));
   };
   const int col_first = first_col(min(blk, cb.total - 1));
 #pragma unroll

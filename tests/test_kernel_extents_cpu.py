@@ -43,3 +43,28 @@ def test_attention_stages_stay_inside_the_fragments(tmp_path):
               }
           }
   return 0;""")
+
+
+def test_projection_columns_stay_inside_the_weight(tmp_path):
+    """Every width up to 1600 columns, also as two ranges of blocks (keys, then
+    values): each block of 48 columns, whole or with groups past the last."""
+    _run(tmp_path, """
+  for (int ksteps : {4, 8, 16, 24})
+    for (int N = 16; N <= 1600; N += 16)
+      for (int n_swap : {0, N / 2 / 16 * 16, N}) {
+        const long bytes = static_cast<long>(N) * ksteps * 64;
+        const int first = (n_swap + 47) / 48, total = first + (N - n_swap + 47) / 48;
+        for (int blk = 0; blk < total; ++blk)
+          for (int j = 0; j < 3; ++j)
+            for (int step = 0; step < ksteps; ++step) {
+              const int col0 = blk < first ? blk * 48 : n_swap + (blk - first) * 48;
+              const long at = column_group_offset(col0, j, N, ksteps, step);
+              const long want = (static_cast<long>(std::min(col0 / 16 + j, N / 16 - 1)) * ksteps + step) * 1024;
+              if (at + 1024 > bytes || at != want) {
+                std::printf("N=%d n_swap=%d block %d group %d step %d: %ld of %ld\\n", N, n_swap, blk, j,
+                            step, at, bytes);
+                return 1;
+              }
+            }
+      }
+  return 0;""")
