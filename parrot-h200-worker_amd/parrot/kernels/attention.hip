@@ -45,6 +45,7 @@
 // The weight fragments are loaded once the key loop is done (the block
 // registers are free then), while the wavefronts' states are merged.
 #include "common.h"
+#include "extents.h"
 
 namespace parrot {
 
@@ -119,9 +120,9 @@ __global__ __launch_bounds__(64 * kAttnWaves) void causal_attention_kernel(AttnA
   const uint16_t* qb = a.q + b * a.qs[0] + h * a.qs[1];
   const int query = q0 + c;
 
-  // K and V^T of this kv head through buffer resources: the per-lane byte
-  // offset is fixed, the block's key offset is uniform (an SGPR), and K rows
-  // past the sequence read as zero.
+  // K and V^T of this kv head through buffer resources: with fragment-order
+  // operands the per-lane byte offset is fixed and the block's offset is
+  // uniform (an SGPR).  Strided K rows past the sequence read its last row.
   const int ks2 = static_cast<int>(a.ks[2]), vs2 = static_cast<int>(a.vs[2]);
   const int nblk = (T + kAttnKeys - 1) / kAttnKeys;
   const int64_t bh = static_cast<int64_t>(b) * a.kv_heads + kvh;
@@ -131,8 +132,8 @@ __global__ __launch_bounds__(64 * kAttnWaves) void causal_attention_kernel(AttnA
   const __amdgpu_buffer_rsrc_t v_rsrc =
       FRAG ? make_rsrc(a.vt + bh * nblk * (kAttnKeys * D), static_cast<uint32_t>(nblk) * kAttnKeys * D * 2)
            : make_rsrc(a.vt + b * a.vs[0] + kvh * a.vs[1], static_cast<uint32_t>(D) * vs2 * 2);
-  const uint32_t k_off0 = FRAG ? lane * 16 : static_cast<uint32_t>(c * ks2 + 8 * g) * 2;
-  const uint32_t k_off1 = FRAG ? k_off0 + KS * 1024 : k_off0 + static_cast<uint32_t>(16 * ks2) * 2;
+  const uint32_t k_off0 = FRAG ? lane * 16 : 16 * g;
+  const uint32_t k_off1 = k_off0 + KS * 1024;  // (fragment order)
   const uint32_t v_off = FRAG ? lane * 16 : static_cast<uint32_t>(c * vs2 + 4 * g) * 2;
 
   // Q^T as the B operand: lane holds query q0 + c, dims 32 s + 8 g .. +8.
@@ -179,11 +180,12 @@ __global__ __launch_bounds__(64 * kAttnWaves) void causal_attention_kernel(AttnA
       }
       return;
     }
-    const uint32_t ko = static_cast<uint32_t>(k0) * ks2 * 2;
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      x.k[0][s] = __builtin_bit_cast(bf16x8, buffer_load16(k_rsrc, k_off0 + 64 * s, ko));
-      x.k[1][s] = __builtin_bit_cast(bf16x8, buffer_load16(k_rsrc, k_off1 + 64 * s, ko));
+    for (int n = 0; n < 2; ++n) {
+      const uint32_t row = k_off0 + key_row_offset(k0 + 16 * n + c, T, ks2);
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+        x.k[n][s] = __builtin_bit_cast(bf16x8, buffer_load16(k_rsrc, row + 64 * s, 0));
     }
     // V^T rows hold at least roundup(T, 32) keys, so every block is in
     // range; keys past T are zeroed in `step`.

@@ -25,6 +25,12 @@ PARROT_EXTENT uint32_t stage_piece_offset(int first, int piece, int pieces, int 
   return static_cast<uint32_t>(block * pieces + (second ? piece - pieces : piece)) * 1024u;
 }
 
+// attention.hip, strided K: byte offset of row `key` of a sequence of T rows,
+// `stride` elements apart.
+PARROT_EXTENT uint32_t key_row_offset(int key, int T, int stride) {
+  return static_cast<uint32_t>(key < T ? key : T - 1) * static_cast<uint32_t>(stride) * 2u;
+}
+
 // proj.hip, many rows: byte offset in the packed weight (N columns, ksteps
 // 32-wide k steps) of k step `step` of the 16-column group `group` of the block
 // that starts at column col0.

@@ -68,3 +68,21 @@ def test_projection_columns_stay_inside_the_weight(tmp_path):
             }
       }
   return 0;""")
+
+
+def test_strided_key_rows_stay_inside_the_sequence(tmp_path):
+    """Every 32-key block of every sequence length, packed and padded rows."""
+    _run(tmp_path, """
+  for (int d : {64, 96, 128})
+    for (int stride : {d, 8 * d + 8})
+      for (int T = 1; T <= 300; ++T)
+        for (int k0 = 0; k0 < T; k0 += 32)
+          for (int key = k0; key < k0 + 32; ++key) {
+            const long at = key_row_offset(key, T, stride);
+            const long want = static_cast<long>(std::min(key, T - 1)) * stride * 2;
+            if (at != want || at + d * 2 > (static_cast<long>(T - 1) * stride + d) * 2) {
+              std::printf("d=%d stride=%d T=%d key %d: %ld\\n", d, stride, T, key, at);
+              return 1;
+            }
+          }
+  return 0;""")
