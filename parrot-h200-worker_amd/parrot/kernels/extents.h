@@ -39,4 +39,11 @@ PARROT_EXTENT uint32_t column_group_offset(int col0, int group, int N, int kstep
   return static_cast<uint32_t>((at < last ? at : last) * ksteps + step) * 1024u;
 }
 
+// gemm.hip, persistent tiles: the segment row whose id row r of row tile
+// `tile` (bm rows) takes.
+PARROT_EXTENT int tile_source_row(int tile, int bm, int r, int rows) {
+  const int s = tile * bm + r;
+  return s < rows ? s : rows - 1;
+}
+
 }  // namespace parrot

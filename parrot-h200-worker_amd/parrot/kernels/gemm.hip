@@ -24,7 +24,7 @@
 // the epilogue scales routed rows by their route weight and scatters them
 // to assignment order (fp32), shared rows go to token order (fp32).
 #include "common.h"
-
+#include "extents.h"
 
 namespace parrot {
 
@@ -1148,12 +1148,13 @@ __global__ __launch_bounds__(256, 2) void grouped_gemm_big_kernel(GemmArgs p) {
     return w;
   };
 
-  // Row ids of a routed tile into ids_s[buf] (wavefronts 0 and 1, one row per lane).
+  // Row ids of a routed tile into ids_s[buf] (wavefronts 0 and 1, one row per
+  // lane; rows past the segment's end take its last id, so that every address
+  // made from ids_s is a token's).
   auto load_ids = [&](const Work& w, int buf) {
     if (w.t.seg == E || wave >= kBigRows / kWave) return;
-    const int s = w.t.mt * kBigRows + tid;
+    const int s = tile_source_row(w.t.mt, kBigRows, tid, w.t.rows);
     int* dst = &ids_s[buf][wave * kWave];
-    if (s >= w.t.rows) return;
     if (p.sorted != nullptr) {
       buffer_to_lds4(make_rsrc(p.sorted, static_cast<uint32_t>(T) * 8u), dst,
                      static_cast<uint32_t>(w.t.hbase + s) * 4u);
@@ -1177,7 +1178,8 @@ __global__ __launch_bounds__(256, 2) void grouped_gemm_big_kernel(GemmArgs p) {
                                         : p.w_routed + static_cast<int64_t>(w.t.seg) * w.N * w.K;
     return make_rsrc(base, static_cast<uint32_t>(static_cast<int64_t>(w.N) * w.K * 2));
   };
-  // Rows past the segment's end read some row (or zeros); they are not stored.
+  // Rows past the segment's end read its last row, or other hidden rows, or
+  // zeros past the buffer's end; they are not stored.
   auto block_offsets = [&](const Work& w, int buf, uint32_t (&off)[4]) {
     const int r0 = wave * 32 + (lane & 15);
     int id[2];

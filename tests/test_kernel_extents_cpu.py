@@ -86,3 +86,19 @@ def test_strided_key_rows_stay_inside_the_sequence(tmp_path):
             }
           }
   return 0;""")
+
+
+def test_every_row_of_an_expert_tile_takes_a_row_of_its_segment(tmp_path):
+    """Every segment length, whole tiles and partial last ones: no row of a
+    tile is left without an id of the segment."""
+    _run(tmp_path, """
+  for (int rows = 1; rows <= 700; ++rows)
+    for (int tile = 0; tile * 128 < rows; ++tile)
+      for (int r = 0; r < 128; ++r) {
+        const int s = tile_source_row(tile, 128, r, rows);
+        if (s != std::min(tile * 128 + r, rows - 1)) {
+          std::printf("rows=%d tile %d row %d: %d\\n", rows, tile, r, s);
+          return 1;
+        }
+      }
+  return 0;""")
