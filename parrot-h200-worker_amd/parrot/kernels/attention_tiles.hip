@@ -301,6 +301,16 @@ __global__ __launch_bounds__(256, 2) void attention_tile_kernel(TileArgs a) {
 #pragma unroll
       for (int i = 0; i < DT; ++i)
         o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[2 * i + s], pf[s], o[i], 0, 0, 0);
+    // A block that the tile's last 16 queries have left behind (as they have
+    // every block before it, so their sums are still 0): its weights are 0 for
+    // them, but 0 times an infinite value is not.  Each 16 queries choose their
+    // blocks in attention.hip too.
+    if (k0 + 31 <= q0 + 16 - W) {
+#pragma unroll
+      for (int i = 0; i < DT; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[i][e] = col < 16 ? o[i][e] : 0.0f;
+    }
   };
   constexpr int kNext = kBlockElems * 2;  // bytes from one block to the next
   auto block = [&](uint32_t lds, int k0) {

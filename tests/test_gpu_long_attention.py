@@ -88,3 +88,32 @@ def test_long_attention_non_finite_keys(b):
     assert rows[:, 411:511].all() and not rows[:, 511:].any()
     # two roundings to bf16 apart at most (P, then the output)
     assert (got - old).abs()[~bad].max() <= 2e-2
+
+
+# windows whose lower edge falls inside a block, on its border, and in the
+# middle of a 32-query tile
+@pytest.mark.parametrize("b,window", [(2, 100), (2, 96), (2, 113), (24, 100), (24, 16), (24, 48)])
+def test_long_attention_infinite_values(b, window):
+    """An infinite value row reaches exactly the queries that it reaches in
+    the 16-query kernel: those whose 16 queries see a key of its block."""
+    from parrot import hip_moe
+    H, Hk, t, d = 8, 2, 530, 96
+    print(f"long attention, infinite values, b={b} window={window}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(b + window)
+    q, k, v = (torch.randn(b, h, t, d, generator=g, device="cuda").bfloat16() for h in (H, Hk, Hk))
+    rows = torch.arange(t, device="cuda") // 16 * 16  # each query's 16
+    touched = torch.zeros(b, t, H, d, dtype=torch.bool, device="cuda")
+    for n, h, key, dim, value in ((0, 0, 70, 5, "inf"), (0, 1, 200, 90, "-inf"),
+                                  (b - 1, 0, 383, 33, "inf")):
+        v[n, h, key, dim] = float(value)
+        block = key // 32 * 32
+        sees = (block <= rows + 15) & (block + 31 > rows - window)
+        touched[n, :, h * (H // Hk):(h + 1) * (H // Hk), dim] |= sees[:, None]
+    kf, vf = _fragments(hip_moe, k, v)
+    with torch.no_grad():
+        got = hip_moe.causal_attention_frag(q, kf, vf, kv_heads=Hk, scale=d ** -0.5, window=window)
+        old = hip_moe.causal_attention(q, k, v, scale=d ** -0.5, window=window)
+    for out in (old, got):
+        assert torch.equal(~torch.isfinite(out).view(b, t, H, d), touched)
+    fine = torch.isfinite(old)
+    assert (got - old).abs()[fine].max() <= 2e-2  # as for the non-finite keys
