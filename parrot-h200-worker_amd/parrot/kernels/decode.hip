@@ -423,12 +423,10 @@ __global__ __launch_bounds__(256) void decode_split_kernel(
   // Every load first: this wavefront's 16 keys, the query heads, the values.
   const int g = lane >> 4, c = lane & 15;
   bf16x8 kf[KS];
-  {
-    const uint16_t* kr = row(kc, kn, c0 + 16 * wave + c) + 8 * g;
+  const uint16_t* kr = row(kc, kn, c0 + 16 * wave + c) + 8 * g;
 #pragma unroll
-    for (int s = 0; s < KS; ++s)
-      kf[s] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(kr + 32 * s));
-  }
+  for (int s = 0; s < KS; ++s)
+    kf[s] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(kr + 32 * s));
   const QT* qrow = q + (static_cast<int64_t>(b) * heads + kvh * rep + min(c, rep - 1)) * D + 8 * g;
   uint4 vr[kPieces];
 #pragma unroll
@@ -444,6 +442,24 @@ __global__ __launch_bounds__(256) void decode_split_kernel(
 #pragma unroll
     for (int t = kParts - 1; t >= 0; --t)  // small parts first
       sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(part[t], kf[s], sc, 0, 0, 0);
+  }
+  if constexpr (kParts > 1) {
+    // An infinite key makes NaN of a later part that is 0 or of the other
+    // sign, where the whole query's product is infinite: a NaN score becomes
+    // the leading parts' sum, which is NaN only if the whole product is.
+    if (__any(sc[0] != sc[0] || sc[1] != sc[1] || sc[2] != sc[2] || sc[3] != sc[3])) {
+      f32x4 lead = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1  // a rare path: the keys are read again and hold no registers
+      for (int s = 0; s < KS; ++s) {
+        bf16x8 part[kParts];
+        query_parts(qrow + 32 * s, c < rep, part);
+        const uint4 key = *reinterpret_cast<const uint4*>(kr + 32 * s);
+        lead = __builtin_amdgcn_mfma_f32_16x16x32_bf16(part[0], __builtin_bit_cast(bf16x8, key), lead,
+                                                       0, 0, 0);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sc[r] = sc[r] == sc[r] ? sc[r] : lead[r];
+    }
   }
   // The chunk that holds `pos` stores the new rows.
   if (c0 + kSplitKeys >= L && tid < D) {

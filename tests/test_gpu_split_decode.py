@@ -118,6 +118,37 @@ def test_split_decode_attention_latent(monkeypatch, b, H, r, position):
     assert err[1] <= max(1e-6, 1.5 * err[0])
 
 
+# in the first chunk and beside the newest latent; queries that are bf16
+# values (no later parts) and such that are not
+@pytest.mark.parametrize("key", [5, 130])
+@pytest.mark.parametrize("rounded", [True, False])
+def test_split_decode_attention_latent_infinite(monkeypatch, key, rounded):
+    """An infinite latent entry takes its key out of the softmax (score -inf)
+    or makes the head NaN (score +inf), as in the one-launch form."""
+    hip_moe = _split_always(monkeypatch)
+    print(f"split latent infinite key {key} rounded={rounded}", flush=True)
+    b, H, r, position, dim = 1, 8, 128, 130, 3
+    g = torch.Generator().manual_seed(key)
+    q = torch.randn(b, 1, H, r, generator=g)
+    q[..., dim] = q[..., dim].abs() + 0.25
+    q[:, :, H // 2:, dim] *= -1  # heads that see -inf, then heads that see +inf
+    q = (q.bfloat16().float() if rounded else q).view(b, 1, H * r).cuda()
+    new = torch.randn(b, 1, r, generator=g).bfloat16().cuda()
+    cache = torch.randn(b, 200, r, generator=g).bfloat16().cuda()
+    (new[:, 0] if key == position else cache[:, key])[:, dim] = float("-inf")
+    pos = torch.tensor([position], dtype=torch.int32, device="cuda")
+    with torch.no_grad():
+        one, got = (hip_moe.decode_attention_latent(q, new, cache.clone(), pos, H, 96 ** -0.5,
+                                                    context=context).view(H, r)
+                    for context in (None, position + 1))
+    for out in (one, got):  # weight 0 times an infinite value: that dimension alone
+        finite = torch.isfinite(out)
+        assert finite[:H // 2, :dim].all() and finite[:H // 2, dim + 1:].all()
+        assert not finite[:, dim].any() and not finite[H // 2:].any()
+    keep = torch.isfinite(one)
+    assert ((one - got).abs()[keep] <= 1e-5).all()  # fp32 sums of ~130 terms of size 1
+
+
 @pytest.mark.parametrize("logits", [False, True])
 def test_decode_graph_crosses_into_the_split_form(logits):
     """Steps on either side of the position from which the keys are split
