@@ -18,11 +18,11 @@
 namespace parrot {
 
 // attention_tiles.hip: byte offset in one kv head's K (or V) fragments, nblk
-// blocks of `pieces` KB, of KB `piece` of the two blocks from `first` on.
+// blocks of `pieces` KB, of KB `piece` of the two blocks from `first` on (of
+// `first` once more where the second is missing).
 PARROT_EXTENT uint32_t stage_piece_offset(int first, int piece, int pieces, int nblk) {
-  const bool second = piece >= pieces;
-  const int block = second && first + 1 < nblk ? first + 1 : first;
-  return static_cast<uint32_t>(block * pieces + (second ? piece - pieces : piece)) * 1024u;
+  const int missing = first + 1 < nblk ? 0 : pieces;
+  return static_cast<uint32_t>(first * pieces + piece - (piece >= pieces ? missing : 0)) * 1024u;
 }
 
 // attention.hip, strided K: byte offset of row `key` of a sequence of T rows,
