@@ -219,6 +219,13 @@ __global__ __launch_bounds__(256, 2) void attention_tile_kernel(TileArgs a) {
   const uint32_t v_off =
       static_cast<uint32_t>(SB * kBlockElems * 2 + (col >> 4) * 1024 + half * 256 + (col & 15) * 16);
 
+  // The first block in which this lane's query sees a key.  Blocks before it,
+  // which other queries of the tile do see, have weight 0 for this one, but 0
+  // times an infinite value is not: its sums start from 0 at that block, in
+  // `raise`, where m = -inf leaves nothing to scale (a check after every block
+  // cost 2-4 %).
+  const int first_seen = max(0, q0 + col - W + 1) & ~31;
+
   // Running maximum m (log2 units) per query, shared by its two lanes and
   // raised only when a score passes it by more than 2^8; each lane sums its
   // own probabilities (see attention.hip).
@@ -256,12 +263,18 @@ __global__ __launch_bounds__(256, 2) void attention_tile_kernel(TileArgs a) {
     for (int i = 0; i < 5; ++i) t[i] = fmaxf(fmaxf(x[3 * i], x[3 * i + 1]), x[3 * i + 2]);
     return fmaxf(fmaxf(fmaxf(t[0], t[1]), t[2]), fmaxf(fmaxf(t[3], t[4]), x[15]));
   };
-  auto raise = [&](float mx) {  // mx: this lane's largest score
+  auto raise = [&](float mx, int k0) {  // mx: this lane's largest score
     mx *= a.scale_log2;
     if (__ballot(mx > m + kLazy) != 0) {
       const float mn = fmaxf(m, fmaxf(mx, __shfl_xor(mx, 32)));
       const float alpha = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mn);
       l *= alpha;
+      if (static_cast<uint32_t>(k0 - first_seen) < 32u * KG) {  // the key group's first such block
+#pragma unroll
+        for (int i = 0; i < DT; ++i)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) o[i][e] = 0.0f;
+      }
 #pragma unroll
       for (int i = 0; i < DT; ++i)
 #pragma unroll
@@ -301,16 +314,6 @@ __global__ __launch_bounds__(256, 2) void attention_tile_kernel(TileArgs a) {
 #pragma unroll
       for (int i = 0; i < DT; ++i)
         o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[2 * i + s], pf[s], o[i], 0, 0, 0);
-    // A block that the tile's last 16 queries have left behind (as they have
-    // every block before it, so their sums are still 0): its weights are 0 for
-    // them, but 0 times an infinite value is not.  Each 16 queries choose their
-    // blocks in attention.hip too.
-    if (k0 + 31 <= q0 + 16 - W) {
-#pragma unroll
-      for (int i = 0; i < DT; ++i)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) o[i][e] = col < 16 ? o[i][e] : 0.0f;
-    }
   };
   constexpr int kNext = kBlockElems * 2;  // bytes from one block to the next
   auto block = [&](uint32_t lds, int k0) {
@@ -320,7 +323,7 @@ __global__ __launch_bounds__(256, 2) void attention_tile_kernel(TileArgs a) {
     __builtin_amdgcn_sched_barrier(0);
     read_values<0>(lds + v_off, vf);
     mask(sc, k0);
-    raise(max16(sc));
+    raise(max16(sc), k0);
     probabilities(sc, pf);
     values(vf, pf, k0);
   };
@@ -351,6 +354,13 @@ __global__ __launch_bounds__(256, 2) void attention_tile_kernel(TileArgs a) {
     constexpr int kState = DT * 16 * kWave;  // floats per wavefront
     static_assert((4 - 4 / KG) * kState * 4 <= NB * kStageElems * 2, "the merge fits the stages");
     float* ob = reinterpret_cast<float*>(&stage[0][0]);
+    const int diag = q0 >> 5;
+    if ((diag - ((diag - lo - kw) & (KG - 1))) * 32 < first_seen) {  // this key group had none
+#pragma unroll
+      for (int i = 0; i < DT; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[i][e] = 0.0f;
+    }
     __syncthreads();  // everybody has read the last stage
     if (kw > 0) {
       const int at = slot * (KG - 1) + kw - 1;

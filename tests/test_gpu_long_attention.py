@@ -94,26 +94,27 @@ def test_long_attention_non_finite_keys(b):
 # middle of a 32-query tile
 @pytest.mark.parametrize("b,window", [(2, 100), (2, 96), (2, 113), (24, 100), (24, 16), (24, 48)])
 def test_long_attention_infinite_values(b, window):
-    """An infinite value row reaches exactly the queries that it reaches in
-    the 16-query kernel: those whose 16 queries see a key of its block."""
+    """An infinite value row reaches exactly the queries that see a key of its
+    32-key block, and no query that it does not reach in the 16-query kernel,
+    where the 16 queries of a workgroup share their blocks."""
     from parrot import hip_moe
     H, Hk, t, d = 8, 2, 530, 96
     print(f"long attention, infinite values, b={b} window={window}", flush=True)
     g = torch.Generator(device="cuda").manual_seed(b + window)
     q, k, v = (torch.randn(b, h, t, d, generator=g, device="cuda").bfloat16() for h in (H, Hk, Hk))
-    rows = torch.arange(t, device="cuda") // 16 * 16  # each query's 16
-    touched = torch.zeros(b, t, H, d, dtype=torch.bool, device="cuda")
+    rows = torch.arange(t, device="cuda")
+    touched, touched16 = torch.zeros(2, b, t, H, d, dtype=torch.bool, device="cuda")
     for n, h, key, dim, value in ((0, 0, 70, 5, "inf"), (0, 1, 200, 90, "-inf"),
                                   (b - 1, 0, 383, 33, "inf")):
         v[n, h, key, dim] = float(value)
-        block = key // 32 * 32
-        sees = (block <= rows + 15) & (block + 31 > rows - window)
-        touched[n, :, h * (H // Hk):(h + 1) * (H // Hk), dim] |= sees[:, None]
+        block, heads = key // 32 * 32, slice(h * (H // Hk), (h + 1) * (H // Hk))
+        for mask, first in ((touched, rows), (touched16, rows // 16 * 16)):
+            mask[n, :, heads, dim] |= ((block <= rows) & (block + 31 > first - window))[:, None]
     kf, vf = _fragments(hip_moe, k, v)
     with torch.no_grad():
         got = hip_moe.causal_attention_frag(q, kf, vf, kv_heads=Hk, scale=d ** -0.5, window=window)
         old = hip_moe.causal_attention(q, k, v, scale=d ** -0.5, window=window)
-    for out in (old, got):
-        assert torch.equal(~torch.isfinite(out).view(b, t, H, d), touched)
+    assert torch.equal(~torch.isfinite(got).view(b, t, H, d), touched)
+    assert torch.equal(~torch.isfinite(old).view(b, t, H, d), touched16)
     fine = torch.isfinite(old)
     assert (got - old).abs()[fine].max() <= 2e-2  # as for the non-finite keys
