@@ -14,7 +14,19 @@ import torch
 from torch import Tensor
 
 from . import hip_moe
-from .model import GenerationState, Parrot
+from .model import GenerationState, LocalKVCache, Parrot
+
+
+def split_forms(start: int, limit: int, batch: int, splits: bool) -> list[tuple[bool, int]]:
+    """The forms of the step (whether its attention splits the keys) that a
+    generation of ``batch`` sequences from position ``start`` to ``limit``
+    comes to, each with the position whose step is captured.  ``splits``: the
+    model has layers that split at all."""
+    if not splits or not hip_moe.decode_splits(limit, batch):
+        return [(False, start)]
+    if hip_moe.decode_splits(start + 1, batch):
+        return [(True, start)]
+    return [(False, start), (True, limit - 1)]
 
 
 class DecodeGraph:
@@ -43,39 +55,59 @@ class DecodeGraph:
         device = state.position_device.device
         self.ids = torch.zeros((state.batch_size, 1), dtype=torch.long, device=device)
         start = state.position
-        if start >= model.config.max_seq_len:
+        limit = model.config.max_seq_len
+        if start >= limit:
             raise ValueError("Generation state has reached max_seq_len")
+        # The step's attention splits the keys of long contexts over workgroups
+        # (hip_moe.decode_splits), a choice of launches made when a graph is
+        # captured: one graph per form that the generation comes to, all captured
+        # here, so that no step waits for a capture or fails in one.  Both forms
+        # are right at every position.
+        self.out: Tensor | None = None
+        self.graphs: dict[bool, torch.cuda.CUDAGraph] = {}
+        forms = split_forms(start, limit, state.batch_size, self._split_layers(limit))
         # One eager step on a side stream fills every lazily built cache
         # (packed weights, absorbed maps, RoPE tables, scratch buffers);
         # its cache row at `start` is rewritten by the first real step.
-        # The step's attention splits the keys of long contexts over workgroups
-        # (hip_moe.decode_splits), a choice of launches made when a graph is
-        # captured: one graph per form, the second captured when the position
-        # first needs it.
-        self.out: Tensor | None = None
-        self.graphs: dict[bool, torch.cuda.CUDAGraph] = {}
-        self._capture(start)
-
-    def _splits(self) -> bool:
-        return hip_moe.decode_splits(self.state.position + 1, self.state.batch_size)
-
-    def _capture(self, start: int) -> None:
-        device = self.ids.device
         side = torch.cuda.Stream(device)
         side.wait_stream(torch.cuda.current_stream(device))
         with torch.cuda.stream(side):
             self._run()
         torch.cuda.current_stream(device).wait_stream(side)
+        for splits, position in forms:
+            # The device position, which the captured launches read, stays what
+            # it is: the host's alone chooses the form.
+            self.state.position = position
+            self._capture(splits)
         self._rewind(start)
+
+    def _split_layers(self, limit: int) -> bool:
+        """Whether any layer splits its keys at the longest context."""
+        c, b = self.model.config, self.state.batch_size
+        return any(
+            hip_moe.decode_split_bytes(b, c.n_heads, c.n_kv_heads, c.head_dim, cache.key.shape[2],
+                                       c.window_size, limit)
+            if isinstance(cache, LocalKVCache) else
+            hip_moe.decode_split_bytes(b, c.n_heads, 1, c.kv_latent_dim, cache.latent.shape[1],
+                                       cache.latent.shape[1], limit)
+            for cache in self.state.layers)
+
+    def _form(self) -> bool:
+        """The captured form that the step at the state's position takes."""
+        splits = hip_moe.decode_splits(self.state.position + 1, self.state.batch_size)
+        return splits if splits in self.graphs else not splits
+
+    def _capture(self, splits: bool) -> None:
         graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph):
+        # One pool for all: the graphs never run at the same time.
+        pool = next(iter(self.graphs.values())).pool() if self.graphs else None
+        with torch.cuda.graph(graph, pool=pool):
             out = self._run()
             if self.out is None:
                 self.out = out
             elif out.data_ptr() != self.out.data_ptr():
                 self.out.copy_(out)  # every graph's output is the same tensor
-        self._rewind(start)
-        self.graphs[self._splits()] = graph
+        self.graphs[splits] = graph
 
     def _run(self) -> Tensor:
         if self.logits:
@@ -97,12 +129,8 @@ class DecodeGraph:
             raise ValueError("decode input must be [cached batch, 1]")
         if self.state.position >= self.model.config.max_seq_len:
             raise ValueError("Generation state has reached max_seq_len")
-        splits = self._splits()
-        if splits not in self.graphs:
-            input_ids = input_ids.clone()  # the eager step may write self.ids
-            self._capture(self.state.position)
         if input_ids.data_ptr() != self.ids.data_ptr():
             self.ids.copy_(input_ids)
-        self.graphs[splits].replay()
+        self.graphs[self._form()].replay()
         self.state.position += 1
         return self.out

@@ -975,15 +975,21 @@ def decode_splits(context: int | None, batch: int, window: int | None = None) ->
     return (context if window is None else min(context, window)) > 320 + 32 * min(batch, 22)
 
 
+def decode_split_bytes(batch: int, heads: int, kv_heads: int, head_dim: int, max_pos: int,
+                       window: int, context: int | None) -> int:
+    """The split form's workspace size, or 0 where the one-launch form runs."""
+    if not decode_splits(context, batch, window):
+        return 0
+    return _abi.load().parrot_decode_attention_split_workspace_bytes(
+        batch, heads, kv_heads, head_dim, max_pos, window)
+
+
 def _split_workspace(q: Tensor, batch: int, heads: int, kv_heads: int, head_dim: int,
                      max_pos: int, window: int, context: int | None) -> Tensor | None:
     """The split form's workspace (a fresh one per call: calls on several
     streams share nothing), or None where the one-launch form runs."""
-    if not decode_splits(context, batch, window) or q.data_ptr() % 16:
-        return None
-    nbytes = _abi.load().parrot_decode_attention_split_workspace_bytes(
-        batch, heads, kv_heads, head_dim, max_pos, window)
-    if nbytes == 0:
+    nbytes = decode_split_bytes(batch, heads, kv_heads, head_dim, max_pos, window, context)
+    if nbytes == 0 or q.data_ptr() % 16:
         return None
     return torch.empty(nbytes, dtype=torch.uint8, device=q.device)
 

@@ -39,3 +39,25 @@ def test_decode_split_arguments():
         return lib.parrot_decode_attention_latent_split_f32(
             q, fake, fake, fake, 1, 8, r, 4096, 0.1, fake, fake, wsb, null)
     assert latent(q=null) == -1 and latent(r=100) == -3 and latent(wsb=64) == -4
+
+
+def test_decode_graph_forms():
+    """The forms a generation comes to, known when its graph is made: none is
+    left to a step, and none is captured that no layer takes."""
+    from parrot.decode_graph import split_forms
+    assert split_forms(128, 4096, 1, True) == [(False, 128), (True, 4095)]
+    assert split_forms(351, 4096, 1, True) == [(False, 351), (True, 4095)]
+    assert split_forms(352, 4096, 1, True) == [(True, 352)]  # its context is 353
+    assert split_forms(128, 352, 1, True) == [(False, 128)]
+    assert split_forms(128, 353, 1, True) == [(False, 128), (True, 352)]
+    assert split_forms(2000, 4096, 1, False) == [(False, 2000)]
+    assert split_forms(800, 1024, 64, True) == [(False, 800)]
+
+
+def test_decode_split_bytes_by_shape():
+    from parrot import hip_moe
+    size = hip_moe.decode_split_bytes
+    assert size(1, 8, 2, 96, 4096, 2048, 353) > 0 and size(1, 8, 2, 96, 4096, 2048, 352) == 0
+    assert size(1, 8, 2, 96, 4096, 256, 4096) == 0  # the window stays below the line
+    assert size(1, 8, 2, 16, 4096, 2048, 4096) == 0 and size(1, 34, 2, 96, 4096, 2048, 4096) == 0
+    assert size(1, 8, 2, 96, 4096, 2048, None) == 0

@@ -178,3 +178,46 @@ def test_decode_graph_crosses_into_the_split_form(logits):
         graph._rewind(first - 1)  # back to the one-launch form: no new capture
     graph.step(ids)
     assert len(graph.graphs) == 2 and state.position == first
+
+
+def _long_model(**fields):
+    from parrot import ModelConfig, Parrot
+    cfg = ModelConfig(**{**dict(vocab_size=512, dim=256, n_layers=4, n_heads=4, n_kv_heads=2,
+                                head_dim=64, kv_latent_dim=64, window_size=512, max_seq_len=512,
+                                n_experts=4, expert_dim=64, shared_expert_dim=64,
+                                moe_backend="grouped_hip", depth_backend="hip",
+                                collect_router_stats=False), **fields})
+    torch.manual_seed(3)
+    return Parrot(cfg).to(device="cuda", dtype=torch.bfloat16).eval()
+
+
+# (max_seq_len, prompt): ends below the line, crosses it, starts past it
+@pytest.mark.parametrize("limit,start,forms", [(300, 40, {False}), (512, 40, {False, True}),
+                                               (512, 400, {True})])
+def test_decode_graph_captures_up_front(monkeypatch, limit, start, forms):
+    """Every form that the generation comes to is captured when the graph is
+    made, in one pool; no step captures, and a state set back below the line
+    goes on with what there is."""
+    from parrot.decode_graph import DecodeGraph
+    print(f"decode graph forms, {start} to {limit}", flush=True)
+    model = _long_model(max_seq_len=limit)
+    prompt = torch.randint(0, 512, (2, start), device="cuda")
+    _, state = model.prefill(prompt)
+    graph = DecodeGraph(model, state)
+    assert set(graph.graphs) == forms and state.position == start
+    assert int(state.position_device) == start
+    assert len({g.pool() for g in graph.graphs.values()}) == 1
+    monkeypatch.setattr(torch.cuda, "graph", None)
+    for position in (limit - 1, start):
+        with torch.inference_mode():
+            graph._rewind(position)
+        graph.step(prompt[:, -1:].clone())
+    assert state.position == start + 1
+
+
+def test_decode_graph_of_a_shape_that_never_splits():
+    from parrot.decode_graph import DecodeGraph
+    print("decode graph, head width 16", flush=True)
+    model = _long_model(head_dim=16, kv_latent_dim=16)
+    _, state = model.prefill(torch.randint(0, 512, (1, 400), device="cuda"))
+    assert set(DecodeGraph(model, state).graphs) == {False}
