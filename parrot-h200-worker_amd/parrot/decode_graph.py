@@ -66,20 +66,25 @@ class DecodeGraph:
         self.out: Tensor | None = None
         self.graphs: dict[bool, torch.cuda.CUDAGraph] = {}
         forms = split_forms(start, limit, state.batch_size, self._split_layers(limit))
-        # One eager step on a side stream fills every lazily built cache
-        # (packed weights, absorbed maps, RoPE tables, scratch buffers);
-        # its cache row at `start` is rewritten by the first real step.
-        side = torch.cuda.Stream(device)
-        side.wait_stream(torch.cuda.current_stream(device))
-        with torch.cuda.stream(side):
-            self._run()
-        torch.cuda.current_stream(device).wait_stream(side)
-        for splits, position in forms:
-            # The device position, which the captured launches read, stays what
-            # it is: the host's alone chooses the form.
-            self.state.position = position
-            self._capture(splits)
-        self._rewind(start)
+        try:
+            # One eager step on a side stream fills every lazily built cache
+            # (packed weights, absorbed maps, RoPE tables, scratch buffers);
+            # its cache row at `start` is rewritten by the first real step.
+            side = torch.cuda.Stream(device)
+            side.wait_stream(torch.cuda.current_stream(device))
+            try:
+                with torch.cuda.stream(side):
+                    self._run()
+            finally:
+                torch.cuda.current_stream(device).wait_stream(side)
+            self._rewind(start)
+            for splits, position in forms:
+                # The device position, which the captured launches read, stays
+                # what it is: the host's alone chooses the form.
+                self.state.position = position
+                self._capture(splits)
+        finally:  # no step has been taken, also where the eager one or a capture raised
+            self._rewind(start)
 
     def _split_layers(self, limit: int) -> bool:
         """Whether any layer splits its keys at the longest context."""

@@ -221,3 +221,33 @@ def test_decode_graph_of_a_shape_that_never_splits():
     model = _long_model(head_dim=16, kv_latent_dim=16)
     _, state = model.prefill(torch.randint(0, 512, (1, 400), device="cuda"))
     assert set(DecodeGraph(model, state).graphs) == {False}
+
+
+# the eager step, the first capture and the second one
+@pytest.mark.parametrize("fails_at", [1, 2, 3])
+def test_decode_graph_that_fails_leaves_the_state(monkeypatch, fails_at):
+    """A constructor that raises has taken no step: eager decoding goes on
+    from the same position with the same tokens."""
+    import copy
+    from parrot.decode_graph import DecodeGraph
+    print(f"decode graph failing at run {fails_at}", flush=True)
+    model = _long_model()
+    prompt = torch.randint(0, 512, (2, 40), device="cuda")
+    with torch.inference_mode():
+        _, state = model.prefill(prompt)
+        other = copy.deepcopy(state)
+        runs, run = [], DecodeGraph._run
+
+        def failing(self):
+            runs.append(run(self))
+            if len(runs) == fails_at:
+                raise RuntimeError("planted on the host")
+            return runs[-1]
+        monkeypatch.setattr(DecodeGraph, "_run", failing)
+        with pytest.raises(RuntimeError, match="planted"):
+            DecodeGraph(model, state)
+        assert len(runs) == fails_at and state.position == 40 and int(state.position_device) == 40
+        mine = theirs = prompt[:, -1:]
+        for _ in range(3):
+            mine, theirs = model.decode_next(mine, state)[0], model.decode_next(theirs, other)[0]
+            assert torch.equal(mine, theirs)
