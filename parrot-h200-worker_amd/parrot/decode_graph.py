@@ -97,6 +97,11 @@ class DecodeGraph:
                                        cache.latent.shape[1], limit)
             for cache in self.state.layers)
 
+    @property
+    def graph(self) -> torch.cuda.CUDAGraph:
+        """The captured step that the next ``step`` replays."""
+        return self.graphs[self._form()]
+
     def _form(self) -> bool:
         """The captured form that the step at the state's position takes."""
         splits = hip_moe.decode_splits(self.state.position + 1, self.state.batch_size)
@@ -136,6 +141,6 @@ class DecodeGraph:
             raise ValueError("Generation state has reached max_seq_len")
         if input_ids.data_ptr() != self.ids.data_ptr():
             self.ids.copy_(input_ids)
-        self.graphs[self._form()].replay()
+        self.graph.replay()
         self.state.position += 1
         return self.out

@@ -207,6 +207,7 @@ def test_decode_graph_captures_up_front(monkeypatch, limit, start, forms):
     assert set(graph.graphs) == forms and state.position == start
     assert int(state.position_device) == start
     assert len({g.pool() for g in graph.graphs.values()}) == 1
+    assert graph.graph is graph.graphs[start == 400]  # the next step's
     monkeypatch.setattr(torch.cuda, "graph", None)
     for position in (limit - 1, start):
         with torch.inference_mode():
