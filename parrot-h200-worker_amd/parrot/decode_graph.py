@@ -74,10 +74,12 @@ class DecodeGraph:
             side.wait_stream(torch.cuda.current_stream(device))
             try:
                 with torch.cuda.stream(side):
-                    self._run()
+                    out = self._run()
             finally:
                 torch.cuda.current_stream(device).wait_stream(side)
             self._rewind(start)
+            # Every graph writes the same output tensor.
+            self.out = torch.empty_like(out) if self.logits else self.ids
             for splits, position in forms:
                 # The device position, which the captured launches read, stays
                 # what it is: the host's alone chooses the form.
@@ -112,16 +114,12 @@ class DecodeGraph:
         # One pool for all: the graphs never run at the same time.
         pool = next(iter(self.graphs.values())).pool() if self.graphs else None
         with torch.cuda.graph(graph, pool=pool):
-            out = self._run()
-            if self.out is None:
-                self.out = out
-            elif out.data_ptr() != self.out.data_ptr():
-                self.out.copy_(out)  # every graph's output is the same tensor
+            self._run()
         self.graphs[splits] = graph
 
     def _run(self) -> Tensor:
         if self.logits:
-            out, _ = self.model.decode_step(self.ids, self.state)
+            out, _ = self.model.decode_step(self.ids, self.state, _out=self.out)
         else:
             # The tokens land in the input buffer, read by the next replay's
             # first launch (the embedding gather), after this step's reads.

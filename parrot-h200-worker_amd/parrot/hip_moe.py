@@ -567,17 +567,24 @@ def decode_experts(module: "MoE", flat: Tensor | None, addend: Tensor | None = N
     return out, indices, weights
 
 
-def vocab_logits(h: Tensor, weight: Tensor) -> Tensor:
+def vocab_logits(h: Tensor, weight: Tensor, out: Tensor | None = None) -> Tensor:
     """fp32 logits ``h @ weight^T`` for bf16 rows h [..., dim] and the tied
     head weight [vocab, dim] (cf. the head F.linear, parrot/model.py:714-715):
     the products of the bf16 operands accumulate in fp32 and the result is
-    written in fp32 (one library GEMM with an fp32 output type)."""
+    written in fp32 (one library GEMM with an fp32 output type).  ``out``: a
+    contiguous fp32 tensor [..., vocab] to write them into and return."""
     _require(h, "HIP vocabulary head")
     if weight.dtype != h.dtype or weight.ndim != 2 or weight.shape[1] != h.shape[-1]:
         raise RuntimeError("head weight must be a [vocab, dim] tensor of h's dtype")
     flat = h.reshape(-1, h.shape[-1])
-    out = torch.mm(flat, weight.t(), out_dtype=torch.float32)
-    return out.view(*h.shape[:-1], weight.shape[0])
+    if out is None:
+        out = torch.mm(flat, weight.t(), out_dtype=torch.float32)
+        return out.view(*h.shape[:-1], weight.shape[0])
+    if out.dtype != torch.float32 or out.device != h.device or not out.is_contiguous() or \
+            out.shape != (*h.shape[:-1], weight.shape[0]):
+        raise RuntimeError("out must be a contiguous fp32 [..., vocab] tensor on h's device")
+    torch.mm(flat, weight.t(), out_dtype=torch.float32, out=out.view(-1, weight.shape[0]))
+    return out
 
 
 def vocab_argmax(h: Tensor, weight: Tensor, advance: Tensor | None = None,

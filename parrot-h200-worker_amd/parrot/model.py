@@ -932,16 +932,17 @@ class Parrot(nn.Module):
                 input_ids.device == self.embedding.weight.device and
                 _hip_inference(self.embedding.weight))
 
-    def _head(self, normed: Tensor) -> Tensor:
+    def _head(self, normed: Tensor, out: Tensor | None = None) -> Tensor:
         """Tied vocabulary head (reference parrot/model.py:714-715).  On the
         HIP backend the logits come out in fp32, never rounded to bf16: a
         bf16 rounding of ~0.5-magnitude logits (ulp 2^-8) ties or swaps
         near-equal top logits, the head's share of greedy-argmax
-        disagreement with the fp32 reference."""
+        disagreement with the fp32 reference.  ``out``: where to write them."""
         if self.config.uses_hip and _hip_inference(normed):
             from . import hip_moe
-            return hip_moe.vocab_logits(normed, self.embedding.weight)
-        return F.linear(normed, self.embedding.weight)
+            return hip_moe.vocab_logits(normed, self.embedding.weight, out)
+        logits = F.linear(normed, self.embedding.weight)
+        return logits if out is None else out.copy_(logits)
 
     def _mixed_input(self, stream: _AttnRes | None, x: Tensor, index: int,
                      norm: RMSNorm) -> Tensor:
@@ -1287,8 +1288,8 @@ class Parrot(nn.Module):
                     _next_token_only: bool = False,
                     _out: Tensor | None = None) -> tuple[Tensor, GenerationState]:
         """Append one token per sequence to an existing generation state.
-        ``_out`` (with ``_next_token_only``): an int64 [batch, 1] tensor the
-        greedy tokens are written into and returned as."""
+        ``_out``: the tensor that the logits, or (with ``_next_token_only``,
+        int64 [batch, 1]) the greedy tokens, are written into and returned as."""
         cfg = self.config
         if self.training:
             raise RuntimeError("decode_step requires model.eval()")
@@ -1354,7 +1355,7 @@ class Parrot(nn.Module):
                                           out=_out)
             advanced = True
         else:
-            logits = self._head(h)
+            logits = self._head(h, None if _next_token_only else _out)
             output = logits.argmax(-1) if _next_token_only else logits
             if _next_token_only and _out is not None:
                 output = _out.copy_(output)

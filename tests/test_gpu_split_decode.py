@@ -252,3 +252,31 @@ def test_decode_graph_that_fails_leaves_the_state(monkeypatch, fails_at):
         for _ in range(3):
             mine, theirs = model.decode_next(mine, state)[0], model.decode_next(theirs, other)[0]
             assert torch.equal(mine, theirs)
+
+
+def test_decode_graph_logits_are_written_in_place(monkeypatch):
+    """Both forms' captured steps end in the same output tensor, with no copy
+    behind the vocabulary product."""
+    from parrot import hip_moe
+    from parrot.decode_graph import DecodeGraph
+    print("decode graph logits in place", flush=True)
+    outs, logits = [], hip_moe.vocab_logits
+
+    def recorded(h, weight, out=None):
+        outs.append(logits(h, weight, out))
+        return outs[-1]
+    monkeypatch.setattr(hip_moe, "vocab_logits", recorded)
+    model = _long_model()
+    _, state = model.prefill(torch.randint(0, 512, (2, 40), device="cuda"))
+    del outs[:]
+    graph = DecodeGraph(model, state, logits=True)
+    assert len(outs) == 3 and len(graph.graphs) == 2  # the eager step, then the captured ones
+    assert all(o.data_ptr() == graph.out.data_ptr() and o.shape == (2, 1, 512) for o in outs[1:])
+    h = torch.randn(2, 1, 256, device="cuda").bfloat16()
+    with torch.no_grad():
+        want = logits(h, model.embedding.weight)
+        out = torch.empty_like(want)
+        assert logits(h, model.embedding.weight, out) is out and torch.equal(out, want)
+        for bad in (out[:1], out.double(), out.cpu(), out.transpose(0, 1)):
+            with pytest.raises(RuntimeError, match="contiguous fp32"):
+                logits(h, model.embedding.weight, bad)
