@@ -440,12 +440,15 @@ hipError_t launch_tile_heads(const TileArgs& a, int batch, hipStream_t s) {
 // workgroups the two take 14.5 and 15.3 us (1 x 1000) or 9.4 and 8.8 us
 // (3 x 333), at 512 11.4 and 10.2 us (2 x 512), at 752 24 and 20 us.  One kv
 // head's fragments must be addressable from every stage's base, the query
-// tiles (32 queries at the least) must fit the grid's y, and a zero scale is
-// left out (scores are masked before they are scaled here).
-bool attention_tiles_apply(int batch, int seq, int heads, int head_dim, float scale) {
+// tiles (32 queries at the least) must fit the grid's y, the output takes 8-byte
+// stores, and a zero scale is left out (scores are masked before they are scaled
+// here).
+bool attention_tiles_apply(int batch, int seq, int heads, int head_dim, float scale,
+                           const uint16_t* out) {
   const int64_t groups = static_cast<int64_t>(batch) * heads * ((seq + 15) / 16);
   return scale != 0.0f && groups > 512 && groups < (int64_t{1} << 31) && seq <= 65535 * 32 &&
-         (static_cast<int64_t>(seq) + 256) * head_dim * 2 < (int64_t{1} << 31);
+         (static_cast<int64_t>(seq) + 256) * head_dim * 2 < (int64_t{1} << 31) &&
+         (reinterpret_cast<uintptr_t>(out) & 7u) == 0;
 }
 
 hipError_t launch_attention_tiles(const uint16_t* q, const uint16_t* k_frag,

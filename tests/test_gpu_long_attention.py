@@ -118,3 +118,27 @@ def test_long_attention_infinite_values(b, window):
     assert torch.equal(~torch.isfinite(old).view(b, t, H, d), touched16)
     fine = torch.isfinite(old)
     assert (got - old).abs()[fine].max() <= 2e-2  # as for the non-finite keys
+
+
+def test_long_attention_output_alignment():
+    """An output that takes no 8-byte stores goes to the 16-query kernel: its
+    bits, and nothing written around it."""
+    import ctypes
+
+    from parrot import _abi, hip_moe
+    b, H, Hk, t, d = 2, 8, 2, 600, 64
+    print("long attention, output at 2 bytes past a boundary", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(7)
+    q, k, v = (torch.randn(b, h, t, d, generator=g, device="cuda").bfloat16() for h in (H, Hk, Hk))
+    kf, vf = _fragments(hip_moe, k, v)
+    n = b * t * H * d
+    buffer = torch.full((n + 8,), 3.0, device="cuda").bfloat16()
+    strides = (ctypes.c_int64 * 3)(*q.stride()[:3])
+    with torch.no_grad():
+        old = hip_moe.causal_attention(q, k, v, scale=d ** -0.5, window=t)
+        _abi.check(_abi.load().parrot_causal_attention_frag_bf16(
+            q.data_ptr(), ctypes.cast(strides, ctypes.c_void_p), kf.data_ptr(), vf.data_ptr(), b, t, H,
+            Hk, d, t, d ** -0.5, buffer.data_ptr() + 2, torch.cuda.current_stream().cuda_stream),
+            "parrot_causal_attention_frag_bf16")
+    assert torch.equal(buffer[1:n + 1], old.flatten())
+    assert (buffer[:1] == 3).all() and (buffer[n + 1:] == 3).all()
