@@ -3,9 +3,9 @@
 // v_mfma_f32_32x32x16_bf16 with K and V shared through LDS.
 //
 // causal_attention_kernel gives a workgroup 16 queries of one head and lets
-// every wavefront read its own key blocks, so each K / V byte that leaves L2
-// feeds 16 queries: 12 KB per 1.6 MFLOP, about 55 bytes per clock and CU at
-// 290 TFLOP/s, the L2's limit.  Here a wavefront owns 32 queries, the four of
+// every wavefront read its own key blocks, so a 12 KB block (32 keys of K and V
+// at D = 96) that leaves L2 serves 0.2 MFLOP: 18 TB/s at the 290 TFLOP/s it
+// reaches on long sequences.  Here a wavefront owns 32 queries, the four of
 // a workgroup cover HW heads that share the kv head, and all of them read the
 // same key blocks from LDS, filled by direct-to-LDS copies (fragment-order K
 // and V are contiguous per block) while the blocks before are computed.
@@ -19,25 +19,37 @@
 //                 {4 g .. + 3, 16 + 4 g .. + 3}, g = 2 s + l / 32, of one
 //                 16-byte piece of the V fragments.
 //
-// What bounds it: per 32 keys and 32 queries a wavefront issues 12 MFMAs (384
-// clocks at D = 96) and ~85 vector instructions, 16 of them exp2 (~540
-// clocks).  Three workgroups per CU, out of step with each other, overlap the
-// two to ~600 clocks a block; a wavefront alone takes ~1180, so a grid's last
-// workgroups and small grids run at half the rate.  Measured and not kept:
-// 64 queries per wavefront (half the LDS reads, two wavefronts per SIMD:
-// 105 against 92 us at 4 x 4096), two blocks interleaved in one wavefront
-// (105 us), eight or sixteen wavefronts on one barrier (their softmaxes
-// collide: 120 and 150 us), deeper rings of stages (no change).
+// Precision: P enters its product as two bf16 parts (16 bits).  The eight
+// wavefronts of causal_attention_kernel have a running maximum each, which makes
+// eight large P of a query exactly 1; with one state (or two) and P rounded to
+// one bf16, an output was 3-5 % further from fp64 than there.  Relative to that
+// kernel's error, 24 x 512 tokens, queries 0.3 / 1 / 3 / 8 / 20 times a normal
+// draw: 0.76 / 0.83 / 0.93 / 0.990 / 0.996.  The six products that this adds to a
+// block's twelve cost 12-28 % (4 x 4096 93 -> 120 us, 2 x 2047 28 -> 34).  With
+// the second part for every other 16 keys only, and the maximum raised by 2^2
+// instead of 2^8, it was 106 and 31 us, but the error 1.001 to 1.004 where few keys
+// dominate.
+//
+// What bounds it: 18 MFMAs (576 clocks at D = 96) and about 125 vector
+// instructions, 16 of them exp2, per 32 keys and 32 queries; three workgroups
+// per CU, out of step with each other, overlap the two in part (4 x 4096 runs at
+// 650 TFLOP/s of visible products, 40 % of the MFMA rate with the second part of
+// P).  A wavefront alone runs at about half the rate, so a grid's last workgroups
+// and small grids wait for the serial chain of the longest queries.  Measured and
+// not kept, before P had two parts: 64 queries per wavefront (half the LDS reads,
+// two wavefronts per SIMD: 105 against 92 us at 4 x 4096), two blocks interleaved
+// in one wavefront (105 us), eight or sixteen wavefronts on one barrier (their
+// softmaxes collide: 120 and 150 us), deeper rings of stages (no change).
 //
 // KG = 2 gives every other block of a stage to a second group of wavefronts,
 // merged through LDS at the end: half the queries per workgroup, twice the
 // workgroups, half the serial chain, at twice the K / V traffic.
 //
-// Measured on MI355X (us, causal_attention_kernel / KG = 1 / KG = 2, 8 heads
-// of 96): 4 x 4096, window 2048, 2 kv heads 262 / 95 / 102 (811 TFLOP/s);
-// 2 x 4096 138 / 58 / 57; 2 x 2047, 8 kv heads, causal 64 / 41 / 29;
-// 1 x 2047 37 / 40 / 26; 2 x 512 11.4 / 13.9 / 10.2; 3 x 333 9.4 / 10.5 /
-// 8.8; 1 x 1000 14.5 / 21.4 / 15.3; 1 x 512 6.7 / 13.3 / 10.0.
+// Measured on MI355X (us in graphs of 20 launches, causal_attention_kernel /
+// KG = 1 / KG = 2, 8 heads of 96, 2 kv heads, window 2048): 4 x 4096 268 / 119 /
+// 121; 3 x 4096 201 / 92 / 94; 2 x 4096 135 / 74 / 68; 16 x 512 80 / 20 / 21;
+// 1 x 2000 32 / 44 / 29; 2 x 520 13.7 / 15.2 / 11.9; 1 x 1050 17.2 / 26.1 / 17.8;
+// 8 kv heads, causal: 2 x 2047 65 / 47 / 33; 1 x 2047 36 / 45 / 30.
 #include "common.h"
 #include "extents.h"
 
@@ -282,20 +294,37 @@ __global__ __launch_bounds__(256, 2) void attention_tile_kernel(TileArgs a) {
       m = mn;
     }
   };
-  auto probabilities = [&](const f32x16& sc, bf16x8 (&pf)[2]) {
+  // P of the block as two bf16 parts (see the top): cut off, not rounded, and the
+  // rest raised by 2^-20 P, because a rest of 0 or below would make NaN of an
+  // infinite value.
+  constexpr float kRaise = 1.0f + 0x1p-20f;
+  auto probabilities = [&](const f32x16& sc, bf16x8 (&pf)[2], bf16x8 (&rest)[2]) {
     // A query that has seen no key yet has m = -inf and only -inf scores:
     // exp2(-inf - 0) = 0.
     const float neg = m == -INFINITY ? 0.0f : -m;
     float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[e], a.scale_log2, neg));
-      sum[e & 3] += p;
-      pf[e >> 3][e & 7] = static_cast<__bf16>(p);
+    for (int s = 0; s < 2; ++s) {
+      uint32_t high[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        uint32_t bits[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const int e = 2 * i + k;
+          const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[8 * s + e], a.scale_log2, neg));
+          sum[e & 3] += p;
+          bits[k] = __float_as_uint(p);
+          rest[s][e] = static_cast<__bf16>(
+              __builtin_fmaf(p, kRaise, -__uint_as_float(bits[k] & 0xffff0000u)));
+        }
+        high[i] = __builtin_amdgcn_perm(bits[1], bits[0], 0x07060302u);  // the upper halves
+      }
+      pf[s] = __builtin_bit_cast(bf16x8, make_uint4(high[0], high[1], high[2], high[3]));
     }
     l += (sum[0] + sum[1]) + (sum[2] + sum[3]);
   };
-  auto values = [&](bf16x8 (&vf)[2 * DT], const bf16x8 (&pf)[2], int k0) {
+  auto values = [&](bf16x8 (&vf)[2 * DT], const bf16x8 (&pf)[2], const bf16x8 (&rest)[2], int k0) {
     // Keys past the sequence: their P is 0, but the padding bytes need not
     // be finite.
     if (k0 + 32 > T) {
@@ -314,18 +343,23 @@ __global__ __launch_bounds__(256, 2) void attention_tile_kernel(TileArgs a) {
 #pragma unroll
       for (int i = 0; i < DT; ++i)
         o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[2 * i + s], pf[s], o[i], 0, 0, 0);
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < DT; ++i)
+        o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[2 * i + s], rest[s], o[i], 0, 0, 0);
   };
   constexpr int kNext = kBlockElems * 2;  // bytes from one block to the next
   auto block = [&](uint32_t lds, int k0) {
-    bf16x8 kf[KU], vf[2 * DT], pf[2];
+    bf16x8 kf[KU], vf[2 * DT], pf[2], rest[2];
     lds_frags<0, 512>(lds + k_off, kf);
     f32x16 sc = scores(kf);
     __builtin_amdgcn_sched_barrier(0);
     read_values<0>(lds + v_off, vf);
     mask(sc, k0);
     raise(max16(sc), k0);
-    probabilities(sc, pf);
-    values(vf, pf, k0);
+    probabilities(sc, pf, rest);
+    values(vf, pf, rest, k0);
   };
 
   const uint32_t lds0 = static_cast<uint32_t>(
@@ -415,9 +449,8 @@ hipError_t launch_tile(const TileArgs& a, int batch, hipStream_t s) {
   return hipGetLastError();
 }
 
-// KG = 1 from three workgroups per CU (the residency it is measured at:
-// 768 of them, 3 x 4096 tokens with 8 heads; at 512, 2 x 4096, both forms
-// take the same time).
+// KG = 1 from three workgroups per CU: at 768 tiles (3 x 4096 tokens with 8
+// heads) 92 against 94 us, at 512 (2 x 4096) 74 against 68.
 constexpr int64_t kOneGroupTiles = 768;
 
 template <int D>
