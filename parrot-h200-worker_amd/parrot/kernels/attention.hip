@@ -435,7 +435,7 @@ hipError_t launch_causal_attention(const uint16_t* q, const uint16_t* k, const u
                                    uint16_t* out, hipStream_t s) {
   if (batch == 0 || seq == 0) return hipSuccess;
   const bool frag = k_strides == nullptr;  // fragment-order K and V
-  if (frag && attention_tiles_apply(batch, seq, heads, head_dim, scale, out))
+  if (frag && attention_tiles_apply(batch, seq, heads, head_dim, window, scale, out))
     return launch_attention_tiles(q, k, vt, q_strides, batch, seq, heads, kv_heads, head_dim,
                                   window, scale, out, s);
   AttnArgs a{};

@@ -469,17 +469,27 @@ hipError_t launch_tile_heads(const TileArgs& a, int batch, hipStream_t s) {
 }  // namespace
 
 // From where causal_attention_kernel's grid (16 queries of a head per
-// workgroup, two workgroups resident per CU) no longer starts at once: at 504
-// workgroups the two take 14.5 and 15.3 us (1 x 1000) or 9.4 and 8.8 us
-// (3 x 333), at 512 11.4 and 10.2 us (2 x 512), at 752 24 and 20 us.  One kv
-// head's fragments must be addressable from every stage's base, the query
+// workgroup, two workgroups resident per CU) no longer starts at once, and its
+// rounds take longer than the serial chain over a query's keys takes here
+// (about 12 us per 1000 keys and 5 to start): the more sequences and heads share
+// the grid, the sooner.  Measured, that kernel / this (us): 16 heads in all, 528
+// workgroups, 520 keys 13.7 / 11.9; 12, 600, 800 keys 15.7 / 14.8; 8, 632, 1250
+// keys 19.3 / 19.9, 728, 1450 keys 21.8 / 22.1, 800, 1600 keys 24.9 / 23.9; 4,
+// 800, 2048 keys 29.9 / 30.4, 900, 2048 keys 33.9 / 30.5, 900, 3600 keys 43.4 /
+// 48.0, 1024, 4096 keys 50.6 / 53.9.  At head width 64 the other kernel's rounds
+// are shorter: 8, 728, 1450 keys 16.6 / 18.9, 904, 1800 keys 21.5 / 23.0; 16, 528,
+// 520 keys 10.9 / 10.1.
+//
+// One kv head's fragments must be addressable from every stage's base, the query
 // tiles (32 queries at the least) must fit the grid's y, the output takes 8-byte
 // stores, and a zero scale is left out (scores are masked before they are scaled
 // here).
-bool attention_tiles_apply(int batch, int seq, int heads, int head_dim, float scale,
+bool attention_tiles_apply(int batch, int seq, int heads, int head_dim, int window, float scale,
                            const uint16_t* out) {
   const int64_t groups = static_cast<int64_t>(batch) * heads * ((seq + 15) / 16);
-  return scale != 0.0f && groups > 512 && groups < (int64_t{1} << 31) && seq <= 65535 * 32 &&
+  const int keys = min(min(seq, window), 3072);
+  const int line = max(512, head_dim == 64 ? 344 + keys / 3 : 384 + keys / 4);
+  return scale != 0.0f && groups > line && groups < (int64_t{1} << 31) && seq <= 65535 * 32 &&
          (static_cast<int64_t>(seq) + 256) * head_dim * 2 < (int64_t{1} << 31) &&
          (reinterpret_cast<uintptr_t>(out) & 7u) == 0;
 }

@@ -574,7 +574,7 @@ hipError_t launch_causal_attention(const uint16_t* q, const uint16_t* k, const u
 bool attention_out_width_supported(int n_out);  // 512, 768, 1024
 // Long sequences (attention_tiles.hip): fragment-order K and V through LDS,
 // shared by the wavefronts of a workgroup.
-bool attention_tiles_apply(int batch, int seq, int heads, int head_dim, float scale,
+bool attention_tiles_apply(int batch, int seq, int heads, int head_dim, int window, float scale,
                            const uint16_t* out);
 hipError_t launch_attention_tiles(const uint16_t* q, const uint16_t* k_frag,
                                   const uint16_t* v_frag, const int64_t* q_strides, int batch,

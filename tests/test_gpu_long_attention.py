@@ -38,6 +38,7 @@ def _fragments(hip_moe, k, v):
 # inside a block and longer than the sequence
 @pytest.mark.parametrize("b,H,Hk,t,d,window,scale", [
     (2, 8, 2, 513, 96, 2048, None), (1, 8, 8, 1025, 96, 4096, None),
+    (1, 8, 8, 1601, 96, 4096, None), (1, 8, 4, 2065, 64, 4096, None),
     (2, 8, 2, 1000, 96, 256, None), (9, 6, 6, 161, 64, 33, None),
     (5, 6, 3, 300, 128, 77, None), (3, 16, 2, 190, 96, 5, None), (2, 9, 3, 490, 64, 490, None),
     (24, 8, 2, 500, 96, 2048, None), (16, 8, 8, 769, 64, 100, None),
