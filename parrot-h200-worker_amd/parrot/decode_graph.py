@@ -10,6 +10,8 @@ parrot/metal_moe.py:182-221 and parrot/model.py:832-925).
 """
 from __future__ import annotations
 
+import bisect
+
 import torch
 from torch import Tensor
 
@@ -17,14 +19,14 @@ from . import hip_moe
 from .model import GenerationState, LocalKVCache, Parrot
 
 
-def split_forms(start: int, limit: int, batch: int, splits: bool) -> list[tuple[bool, int]]:
-    """The forms of the step (whether its attention splits the keys) that a
-    generation of ``batch`` sequences from position ``start`` to ``limit``
-    comes to, each with the position whose step is captured.  ``splits``: the
-    model has layers that split at all."""
-    if not splits or not hip_moe.decode_splits(limit, batch):
+def split_forms(start: int, limit: int, line: int | None) -> list[tuple[bool, int]]:
+    """The forms of the step (whether every layer that ever splits its keys does)
+    that a generation from position ``start`` to ``limit`` comes to, each with
+    the position whose step is captured.  ``line``: the first position of the
+    split form, or None."""
+    if line is None or line >= limit:
         return [(False, start)]
-    if hip_moe.decode_splits(start + 1, batch):
+    if start >= line:
         return [(True, start)]
     return [(False, start), (True, limit - 1)]
 
@@ -59,13 +61,14 @@ class DecodeGraph:
         if start >= limit:
             raise ValueError("Generation state has reached max_seq_len")
         # The step's attention splits the keys of long contexts over workgroups
-        # (hip_moe.decode_splits), a choice of launches made when a graph is
+        # (hip_moe.decode_split_bytes), a choice of launches made when a graph is
         # captured: one graph per form that the generation comes to, all captured
         # here, so that no step waits for a capture or fails in one.  Both forms
         # are right at every position.
         self.out: Tensor | None = None
         self.graphs: dict[bool, torch.cuda.CUDAGraph] = {}
-        forms = split_forms(start, limit, state.batch_size, self._split_layers(limit))
+        self._line = self._split_line(limit)
+        forms = split_forms(start, limit, self._line)
         try:
             # One eager step on a side stream fills every lazily built cache
             # (packed weights, absorbed maps, RoPE tables, scratch buffers);
@@ -88,16 +91,18 @@ class DecodeGraph:
         finally:  # no step has been taken, also where the eager one or a capture raised
             self._rewind(start)
 
-    def _split_layers(self, limit: int) -> bool:
-        """Whether any layer splits its keys at the longest context."""
+    def _split_line(self, limit: int) -> int | None:
+        """The first position from which on every layer that splits its keys at
+        the longest context does; None: no layer ever does."""
         c, b = self.model.config, self.state.batch_size
-        return any(
-            hip_moe.decode_split_bytes(b, c.n_heads, c.n_kv_heads, c.head_dim, cache.key.shape[2],
-                                       c.window_size, limit)
-            if isinstance(cache, LocalKVCache) else
-            hip_moe.decode_split_bytes(b, c.n_heads, 1, c.kv_latent_dim, cache.latent.shape[1],
-                                       cache.latent.shape[1], limit)
-            for cache in self.state.layers)
+        shapes = {(c.n_heads, c.n_kv_heads, c.head_dim, cache.key.shape[2], c.window_size)
+                  if isinstance(cache, LocalKVCache) else
+                  (c.n_heads, 1, c.kv_latent_dim, cache.latent.shape[1], cache.latent.shape[1])
+                  for cache in self.state.layers}
+        lines = [bisect.bisect_left(range(limit), True, key=lambda p: bool(
+            hip_moe.decode_split_bytes(b, *shape, p + 1)))
+            for shape in shapes if hip_moe.decode_split_bytes(b, *shape, limit)]
+        return max(lines, default=None)
 
     @property
     def graph(self) -> torch.cuda.CUDAGraph:
@@ -106,7 +111,7 @@ class DecodeGraph:
 
     def _form(self) -> bool:
         """The captured form that the step at the state's position takes."""
-        splits = hip_moe.decode_splits(self.state.position + 1, self.state.batch_size)
+        splits = self._line is not None and self.state.position >= self._line
         return splits if splits in self.graphs else not splits
 
     def _capture(self, splits: bool) -> None:

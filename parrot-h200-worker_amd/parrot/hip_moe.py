@@ -12,6 +12,7 @@ host and never falls back to another backend: unsupported inputs raise.
 from __future__ import annotations
 
 import ctypes
+import math
 from dataclasses import dataclass
 from typing import TYPE_CHECKING
 
@@ -967,8 +968,10 @@ def _check_position(position: Tensor, device: torch.device) -> None:
 def decode_splits(context: int | None, batch: int, window: int | None = None) -> bool:
     """Whether decode attention over ``context`` positions (the new one
     included; None: unknown) splits its keys over workgroups and merges (two
-    launches) instead of streaming them through one workgroup per head.  Both
-    forms are right at every position: the choice is one of speed.
+    launches) instead of streaming them through one workgroup per head, for
+    shapes like the default ones (four to eight query heads per key row; see
+    ``decode_split_line`` for others).  Both forms are right at every
+    position: the choice is one of speed.
 
     The split form's time hardly depends on the context, but grows with the
     batch (its launch covers the whole window), so the line does too.
@@ -982,10 +985,34 @@ def decode_splits(context: int | None, batch: int, window: int | None = None) ->
     return (context if window is None else min(context, window)) > 320 + 32 * min(batch, 22)
 
 
+def decode_split_line(batch: int, heads: int, kv_heads: int, head_dim: int) -> float:
+    """Keys from which the split form is the faster one for a shape.
+
+    It reads a key row once for all the query heads that share it, where the
+    other form reads it once per head; with one to three heads per row that is
+    little, and past a few hundred (sequence, kv head) pairs the other form
+    fills the chip by itself.  Rows of 64 values and less are short pieces.
+    Measured on MI355X in graphs (one launch / split, us): 8 heads, 8 kv heads
+    of 96, b = 1 450 keys 9.0 / 8.9, b = 8 1500 24.4 / 20.4, b = 32 4000
+    89 / 135; 32 of 128, b = 2 1000 24 / 21, b = 8 4000 107 / 158; 32 heads on 8
+    of 128, b = 4 448 12.0 / 18.8, 1000 26 / 21; 4 on 2 of 64, b = 2 1500
+    16.4 / 16.6; latents of 64 b = 4 1500 16.0 / 16.7, 2500 24.5 / 18.  Of 1822
+    measured points the 746 past these lines are all as fast or faster."""
+    pairs = batch * kv_heads
+    if head_dim < 96:
+        return 704 + 640 * math.log2(max(pairs, 1))
+    if heads < 4 * kv_heads:
+        return 320 + 28 * pairs
+    # (more than eight heads per row: four of them in each wavefront)
+    weight = max(1, kv_heads // 2) * (2 if heads > 8 * kv_heads else 1)
+    return 320 + 32 * min(batch * weight, 22)
+
+
 def decode_split_bytes(batch: int, heads: int, kv_heads: int, head_dim: int, max_pos: int,
                        window: int, context: int | None) -> int:
     """The split form's workspace size, or 0 where the one-launch form runs."""
-    if not decode_splits(context, batch, window):
+    if not decode_splits(context, batch, window) or \
+            min(context, window) <= decode_split_line(batch, heads, kv_heads, head_dim):
         return 0
     return _abi.load().parrot_decode_attention_split_workspace_bytes(
         batch, heads, kv_heads, head_dim, max_pos, window)

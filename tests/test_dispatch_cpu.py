@@ -45,13 +45,12 @@ def test_decode_graph_forms():
     """The forms a generation comes to, known when its graph is made: none is
     left to a step, and none is captured that no layer takes."""
     from parrot.decode_graph import split_forms
-    assert split_forms(128, 4096, 1, True) == [(False, 128), (True, 4095)]
-    assert split_forms(351, 4096, 1, True) == [(False, 351), (True, 4095)]
-    assert split_forms(352, 4096, 1, True) == [(True, 352)]  # its context is 353
-    assert split_forms(128, 352, 1, True) == [(False, 128)]
-    assert split_forms(128, 353, 1, True) == [(False, 128), (True, 352)]
-    assert split_forms(2000, 4096, 1, False) == [(False, 2000)]
-    assert split_forms(800, 1024, 64, True) == [(False, 800)]
+    assert split_forms(128, 4096, 352) == [(False, 128), (True, 4095)]
+    assert split_forms(351, 4096, 352) == [(False, 351), (True, 4095)]
+    assert split_forms(352, 4096, 352) == [(True, 352)]
+    assert split_forms(128, 352, 352) == [(False, 128)]
+    assert split_forms(128, 353, 352) == [(False, 128), (True, 352)]
+    assert split_forms(2000, 4096, None) == [(False, 2000)]
 
 
 def test_decode_split_bytes_by_shape():
@@ -61,3 +60,18 @@ def test_decode_split_bytes_by_shape():
     assert size(1, 8, 2, 96, 4096, 256, 4096) == 0  # the window stays below the line
     assert size(1, 8, 2, 16, 4096, 2048, 4096) == 0 and size(1, 34, 2, 96, 4096, 2048, 4096) == 0
     assert size(1, 8, 2, 96, 4096, 2048, None) == 0
+
+
+def test_decode_split_line_by_shape():
+    """The default layers' line, whatever the batch, and later ones where fewer
+    heads share a key row, rows are short, or the pairs are many."""
+    from parrot import hip_moe
+    size, line = hip_moe.decode_split_bytes, hip_moe.decode_split_line
+    for b in (1, 2, 8, 22, 23, 64):
+        first = next(c for c in range(1, 2049) if hip_moe.decode_splits(c, b))
+        for shape in ((8, 2, 96, 4096, 2048), (8, 1, 128, 4096, 4096)):
+            assert size(b, *shape, first) > 0 and size(b, *shape, first - 1) == 0
+    assert size(1, 8, 8, 96, 4096, 4096, 544) == 0 and size(1, 8, 8, 96, 4096, 4096, 545) > 0
+    assert size(8, 32, 32, 128, 4096, 4096, 4096) == 0  # 256 pairs fill the chip
+    assert size(2, 4, 2, 64, 4096, 4096, 1984) == 0 and size(2, 4, 2, 64, 4096, 4096, 1985) > 0
+    assert line(1, 16, 1, 128) == 384 and line(4, 32, 8, 128) == 832

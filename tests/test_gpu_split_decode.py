@@ -11,6 +11,7 @@ def _split_always(monkeypatch):
     from parrot import hip_moe
     monkeypatch.setattr(hip_moe, "decode_splits", lambda context, batch, window=None:
                         context is not None)
+    monkeypatch.setattr(hip_moe, "decode_split_line", lambda *shape: 0)
     return hip_moe
 
 
@@ -181,8 +182,10 @@ def test_decode_graph_crosses_into_the_split_form(logits):
     equal eager steps, and the graph's output stays the same tensor."""
     from parrot import ModelConfig, Parrot, hip_moe
     from parrot.decode_graph import DecodeGraph
-    cfg = ModelConfig(vocab_size=512, dim=256, n_layers=4, n_heads=4, n_kv_heads=2, head_dim=64,
-                      kv_latent_dim=64, window_size=512, max_seq_len=512, n_experts=4,
+    # four heads per key row and rows of 96 and 128: shapes that split at the first
+    # line (four heads of 64 on two would not below 2000 keys)
+    cfg = ModelConfig(vocab_size=512, dim=256, n_layers=4, n_heads=8, n_kv_heads=2, head_dim=96,
+                      kv_latent_dim=128, window_size=512, max_seq_len=512, n_experts=4,
                       expert_dim=64, shared_expert_dim=64, moe_backend="grouped_hip",
                       depth_backend="hip", collect_router_stats=False)
     torch.manual_seed(3)
@@ -208,8 +211,8 @@ def test_decode_graph_crosses_into_the_split_form(logits):
 
 def _long_model(**fields):
     from parrot import ModelConfig, Parrot
-    cfg = ModelConfig(**{**dict(vocab_size=512, dim=256, n_layers=4, n_heads=4, n_kv_heads=2,
-                                head_dim=64, kv_latent_dim=64, window_size=512, max_seq_len=512,
+    cfg = ModelConfig(**{**dict(vocab_size=512, dim=256, n_layers=4, n_heads=8, n_kv_heads=2,
+                                head_dim=96, kv_latent_dim=128, window_size=512, max_seq_len=512,
                                 n_experts=4, expert_dim=64, shared_expert_dim=64,
                                 moe_backend="grouped_hip", depth_backend="hip",
                                 collect_router_stats=False), **fields})
@@ -242,12 +245,35 @@ def test_decode_graph_captures_up_front(monkeypatch, limit, start, forms):
     assert state.position == start + 1
 
 
-def test_decode_graph_of_a_shape_that_never_splits():
+# widths without a split kernel, and a line past the longest context
+@pytest.mark.parametrize("fields", [dict(head_dim=16, kv_latent_dim=16),
+                                    dict(head_dim=64, kv_latent_dim=64)])
+def test_decode_graph_of_a_shape_that_never_splits(fields):
     from parrot.decode_graph import DecodeGraph
-    print("decode graph, head width 16", flush=True)
-    model = _long_model(head_dim=16, kv_latent_dim=16)
+    print(f"decode graph {fields}", flush=True)
+    model = _long_model(**fields)
     _, state = model.prefill(torch.randint(0, 512, (1, 400), device="cuda"))
     assert set(DecodeGraph(model, state).graphs) == {False}
+
+
+def test_decode_graph_between_two_lines():
+    """Layers that split from different positions: the second form begins
+    where the last of them does, and steps equal eager ones on both sides."""
+    import copy
+    from parrot.decode_graph import DecodeGraph
+    print("decode graph, local line 545, latent line 353", flush=True)
+    model = _long_model(n_kv_heads=8, window_size=1024, max_seq_len=1024)
+    prompt = torch.randint(0, 512, (1, 541), device="cuda")
+    with torch.inference_mode():
+        _, state = model.prefill(prompt)
+        other = copy.deepcopy(state)
+        graph = DecodeGraph(model, state)
+        assert set(graph.graphs) == {False, True} and graph._line == 544
+        mine = theirs = prompt[:, -1:].clone()
+        for _ in range(6):
+            mine = graph.step(mine)
+            theirs, other = model.decode_next(theirs, other)
+            assert torch.equal(mine, theirs)
 
 
 # the eager step, the first capture and the second one
