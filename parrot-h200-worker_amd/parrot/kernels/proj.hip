@@ -718,11 +718,30 @@ int row_tiles(const ProjArgs& a, int bm) {
 // us, output 15.3 -> 12.6 us); 64 beyond, for half the weight traffic (2 x
 // 4096: 35.7 -> 31.3 and 22.9 -> 20.7 us).
 constexpr int kRows32 = 4096;
-// From where the tiles beat proj_kernel (16 x 64 per workgroup; us, that
-// kernel / this): q|k|v 768 rows 9.7 / 9.5, 999 rows 11.7 / 9.5; values and
-// keys from the latent 768 rows 5.3 / 5.3, 999 rows 6.6 / 5.9; the plain
-// output 999 rows 7.1 / 7.3, 1024 rows 7.2 / 7.4, 1500 rows 9.7 / 8.4.
+// From where the tiles beat proj_kernel (16 x 64 per workgroup): a number of
+// rows, and of products, since a workgroup here loads its whole A tile first and
+// has eight wavefronts to feed with 48-column blocks, which few columns do not
+// (hence the growth below a few hundred), and since 8-byte stores and the
+// addend's loads weigh more the shorter the k loop is.  Measured in graphs, us,
+// that kernel / this.  Plain, K = 768: 1100 x 768 7.9 / 7.0, 1536 x 512 7.5 / 7.4,
+// 4096 x 256 8.6 / 8.0, 8192 x 128 8.3 / 9.6, 16384 x 128 14.8 / 9.9; K = 512:
+// 1100 x 768 6.4 / 6.4, 4200 x 256 7.1 / 7.7; K = 256: 2048 x 768 6.0 / 6.3, 4096 x
+// 768 8.5 / 8.1, with an addend 9.1 / 9.1, 8192 x 512 12.8 / 10.3; K = 128: 4096 x
+// 1152 9.2 / 8.9, with an addend 9.6 / 10.1, 8192 x 1536 19.4 / 18.4.  Per sequence:
+// q|k|v K = 768 960 x 1152 9.7 / 9.5, K = 512 1024 x 768 7.3 / 8.8, K = 256 2000 x
+// 512 6.9 / 8.3; keys and values from a latent of 128, 999 x 1536 6.6 / 5.9, 980 x
+// 1536 (7 x 140) 5.8 / 6.2, 2000 x 512 4.8 / 5.2.
 constexpr int kRowsFrom = 960, kStoreRowsFrom = 1100;
+
+template <int EPI>
+bool enough_products(const ProjArgs& a) {
+  const double m = 1e6;
+  double need;  // multiply-adds, at very many columns
+  if (EPI != kStore) need = a.K == 128 ? 170 * m : a.K == 256 ? 280 * m : a.K == 512 ? 430 * m : 560 * m;
+  else need = a.K == 128 ? 400 * m : a.K == 256 ? 500 * m : a.K == 512 ? 400 * m : 560 * m;
+  if (EPI == kStore && a.addend != nullptr) need *= a.K == 128 ? 2.7 : a.K == 256 ? 1.7 : 1.0;
+  return static_cast<double>(a.rows) * a.N * a.K >= need * (1.0 + 128.0 / a.N);
+}
 
 template <int EPI>
 bool rows_apply(const ProjArgs& a) {
@@ -730,6 +749,7 @@ bool rows_apply(const ProjArgs& a) {
   if (a.K % 32 || (steps != 4 && steps != 8 && steps != 16 && steps != 24)) return false;
   // 8-byte accesses of the row-major operands and outputs
   const auto aligned8 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; };
+  if (!enough_products<EPI>(a)) return false;
   if (EPI == kStore)
     return a.rows >= kStoreRowsFrom && a.ldo % 4 == 0 && aligned8(a.out) &&
            (a.addend == nullptr || (a.ld_addend % 4 == 0 && aligned8(a.addend)));

@@ -21,7 +21,11 @@ def _operands(rows, k, n, seed, pad=0):
 @pytest.mark.parametrize("rows,k,n,with_addend,pad", [
     (1100, 768, 768, True, 0), (2047, 768, 896, False, 0), (4096, 512, 64, True, 0),
     (4097, 768, 768, True, 0), (4200, 128, 1536, False, 768), (5001, 256, 16, True, 8),
-    (1729, 768, 80, True, 0), (9000, 768, 1152, False, 0)])
+    (1729, 768, 80, True, 0), (9000, 768, 1152, False, 0),
+    # few columns and short k loops change over later: a partial last block of
+    # 16 columns, one block and a part, two, and ten with an addend
+    (1500, 768, 784, True, 0), (24001, 768, 80, True, 8), (37000, 512, 64, False, 0),
+    (9001, 256, 512, True, 0)])
 def test_proj_rows(rows, k, n, with_addend, pad):
     from parrot import hip_moe
     print(f"proj rows={rows} k={k} n={n} addend={with_addend} pad={pad}", flush=True)
