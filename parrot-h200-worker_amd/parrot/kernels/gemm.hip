@@ -1656,12 +1656,27 @@ hipError_t launch_wide(int phase, const GemmArgs& args, int n_max, hipStream_t s
   return hipGetLastError();
 }
 
-// Whether the persistent kernel takes a wide launch: long enough k loops and
-// buffers that 32-bit offsets reach.
+// Whether the persistent kernel takes a wide launch: enough tiles (its 128 x 256
+// ones are half as many as the 128 x 128 kernel's, and below that the chip is half
+// empty), long enough k loops, and buffers that 32-bit offsets reach.  Measured,
+// the layer on 128 x 128 / persistent tiles (us): down only, 96 tiles (8 experts,
+// 1024 tokens, 768/512/256) 42.2 / 43.8, 108 (1200 tokens, 768/1024/512) 56.1 /
+// 58.0, 192 (16 experts, 2048 tokens, 768/512/256) 59.1 / 54.7; both,
+// 2 experts and 600 tokens of 1024/1024/1024 (gate/up 128 tiles, down 64) 54.9 /
+// 57.5, and 54.3 with down on 128 x 128; 4 experts and 1024 tokens of 768/1024/512
+// (192 and 84) 59.7 / 55.6, and 51.9 with down on 128 x 128.
+constexpr int kTilesGateUp = 96, kTilesDown = 160;
+
 bool persistent_applies(int phase, const GemmArgs& a) {
   constexpr int64_t kReach = 0xfffffff0;  // the kernel's offset for dropped stores
   const int k_min = phase == 1 ? a.dim : min(a.hidden_dim, a.shared_dim);
-  return k_min >= kBigKMin && int64_t{6} * a.tokens * a.hstride < kReach &&
+  const int64_t routed_m = 2 * a.tokens / kBigRows + a.experts;
+  const int64_t shared_m = (a.tokens + kBigRows - 1) / kBigRows;
+  const auto columns = [](int n) { return (n + kBigCols - 1) / kBigCols; };
+  const int64_t tiles = phase == 1 ? routed_m * columns(2 * a.hidden_dim) + shared_m * columns(2 * a.shared_dim)
+                                   : (routed_m + shared_m) * columns(a.dim);
+  return tiles >= (phase == 1 ? kTilesGateUp : kTilesDown) && k_min >= kBigKMin &&
+         int64_t{6} * a.tokens * a.hstride < kReach &&
          int64_t{4} * a.tokens * a.dim < kReach &&
          int64_t{4} * a.experts * a.capacity < kReach &&
          int64_t{4} * a.dim * a.hstride < kReach;

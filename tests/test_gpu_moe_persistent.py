@@ -12,11 +12,13 @@ pytestmark = pytest.mark.gpu
 
 # (tokens, experts, dim, hidden, shared, router bias): the smallest k loops and
 # rows per expert, columns that end within a tile, an expert without rows, rows
-# past the grouping's capacity, more tiles than workgroups, partial row tiles
+# past the grouping's capacity, more tiles than workgroups, partial row tiles, and
+# too few tiles for one product or both (128 x 128 tiles there)
 @pytest.mark.parametrize("tokens,experts,dim,hidden,shared,bias", [
     (1025, 4, 256, 256, 256, None), (2048, 16, 768, 512, 256, None),
     (1100, 3, 320, 448, 320, (9.0, 9.0, -90.0)), (4099, 5, 768, 512, 256, (4.0, 2.0, 0.0, 0.0, 0.0)),
     (513, 2, 512, 320, 704, None), (8200, 32, 256, 320, 256, None), (20001, 16, 768, 512, 256, None),
+    (3000, 3, 768, 448, 320, (9.0, 9.0, -90.0)), (1200, 8, 768, 512, 256, None),
     # k loops under 256 in both products, in the second only (its shared, its
     # routed rows): even and skewed segments with partial last tiles
     (4099, 5, 192, 128, 64, (4.0, 2.0, 0.0, 0.0, 0.0)), (1100, 3, 64, 192, 192, (9.0, 9.0, -90.0)),
