@@ -315,7 +315,8 @@ hipError_t launch_decode(const QT* q, const uint16_t* k_new, const uint16_t* v_n
 //
 // One workgroup per (head, sequence) streams the whole window through one
 // CU: 28.8 us at 2048 keys (b = 1), 31.6 us (b = 8) and 65 us for the latent
-// layers at 3900 keys (b = 4), for 0.8-4 MB that the chip reads in 1-2 us.
+// layers at 3900 keys (b = 4), for 1.6, 12.6 and 4 MB of keys and values that the
+// chip reads from HBM in 0.3, 2.4 and 0.8 us.
 // Here a workgroup takes kSplitKeys = 64 consecutive keys of one kv head for
 // all the query heads that share it, so each row is read once (not once per
 // head), and leaves (max, sum, unnormalised output) per head in a workspace;
@@ -420,7 +421,10 @@ __global__ __launch_bounds__(256) void decode_split_kernel(
     return key == pos ? fresh : cache + static_cast<int64_t>(key) * D;
   };
 
-  // Every load first: this wavefront's 16 keys, the query heads, the values.
+  // This wavefront's 16 keys, then its share of the values, then the query heads.
+  // The keys' loads are in flight together; at head widths from 96 on the compiler
+  // keeps `vr` in scratch memory (64 to 144 bytes per lane), so each value piece is
+  // waited for, stored and read back, and each k step waits for its query load.
   const int g = lane >> 4, c = lane & 15;
   bf16x8 kf[KS];
   {

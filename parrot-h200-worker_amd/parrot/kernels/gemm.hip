@@ -988,18 +988,19 @@ void grouped_gemm_wide_kernel(GemmArgs p) {
 // to 324 us, both together to 313.  Four k steps ahead and a ring of five, then,
 // 316 us; raised wave priority around the products 319 us.
 //
-// Measured on MI355X at 32768 tokens, 16 experts (a graph of 10 launches, one
-// workgroup per 128 x 128 tile / persistent, weights through LDS and tiles in
-// turn): gate/up 211 / 147 us, down 133 / 89 us; 65536 tokens 373 / 281 and
-// 276 / 204; 16384 tokens 119 / 85 and 76 / 49.  The form here against that one
-// (kernel trace of the eager layer, 32768 tokens): gate/up 156 -> 139 us
-// (0.93 PFLOP/s), down 103 -> 98 us; 4096 skewed tokens, 32 experts, down
-// 23.3 -> 22.0 us.
+// Measured on MI355X, 16 experts of the default widths (kernel trace of 16 eager
+// layers, median; one workgroup per tile, 128 x 128 or for down from 32768 tokens
+// 256 x 256 / this kernel): 16384 tokens gate/up 114 / 78 us, down 85 / 44; 32768
+// tokens 231 / 165 and 163 / 108 (the fastest of the 16: 200 / 140 and 143 / 90);
+// 65536 tokens 402 / 319 and 292 / 209.  The clock falls over such a run: single
+// layers with pauses between them take 139 and 98 us at 32768 tokens (0.93 PFLOP/s
+// of gate/up).
 //
-// 256 x 256 tiles in one workgroup of eight wavefronts per CU (weights through
-// LDS), in step or half a stage apart: gate/up 157-166 and down 92-97 us where
-// 128 x 256 tiles took 147 and 89.  Copies issued after a stage's first
-// products instead of before: 168 -> 162 there.
+// Not kept, with the weights still through LDS and the tiles in turn (graphs of 10
+// launches): 256 x 256 tiles in one workgroup of eight wavefronts per CU, in step
+// or half a stage apart, gate/up 157-166 and down 92-97 us where 128 x 256 tiles
+// took 147 and 89.  Copies issued after a stage's first products instead of
+// before: 168 -> 162 there.
 constexpr int kBigRows = 128;
 constexpr int kBigCols = 256;
 constexpr int kBigK = 32;       // k values per stage
@@ -1736,13 +1737,13 @@ enum class TilePlan { kStream16, kStream32, kStream64, kWide };
 
 // Average rows per expert from which the wide-MFMA tiles take over, per
 // phase.  They run on the persistent kernel, or where persistent_applies says
-// no on 128 x 128 tiles.  Measured on MI355X, streaming / persistent: down at
-// 256 rows per expert (T = 2048, E = 16) 18.4 / 17.3 us, (T = 4096, E = 32)
-// 28.6 / 22.8, and with two of the 32 experts holding ~95 % of the rows
-// 30.6 / 24.4.  Gate/up there 23.0 / 22.1, 40.8 / 33.9 and 31.8 / 31.0 us, but
+// no on 128 x 128 tiles.  Measured on MI355X (kernel trace), streaming /
+// persistent: down at 256 rows per expert (T = 2048, E = 16) 19.3 / 14.8 us, (T =
+// 4096, E = 32) 34.7 / 18.8, and with two of the 32 experts holding ~95 % of the
+// rows 33.4 / 21.8.  Gate/up there 22.6 / 20.0, 40.5 / 29.2 and 31.9 / 30.2 us, but
 // streaming tiles group the rows themselves and the others need the grouping
-// launches first (7-10 us), so gate/up changes over at 512: T = 2048, E = 8
-// 26.9 -> 21.5 us; T = 4096, E = 16 37.9 -> 30.8 us.
+// launches first (7-10 us), so gate/up changes over at 512: T = 2048, E = 8 22.0 /
+// 20.1 us; T = 4096, E = 16 39.1 / 29.0 us.
 constexpr int64_t kWideRowsGateUp = 512;
 constexpr int64_t kWideRowsDown = 256;
 
