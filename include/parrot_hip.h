@@ -475,7 +475,10 @@ int parrot_causal_attention_bf16(const void* q, const void* k, const void* vt,
  * Keys past seq in the last block may hold anything.  Every fragment of a
  * key block is then one contiguous 1 KB load (row-major K and V^T loads
  * touch 16 rows per instruction, which bounds the strided entry point at
- * prefill sizes).  Same results as parrot_causal_attention_bf16. */
+ * prefill sizes).  Same results as parrot_causal_attention_bf16 up to the
+ * order of fp32 sums and the rounding of P: long sequences run on a kernel of
+ * their own, whose P has two bf16 parts (no larger an error against fp64).
+ * The same bits where batch * heads * ceil(seq / 16) <= 512. */
 int parrot_causal_attention_frag_bf16(const void* q, const int64_t* q_strides, const void* k_frag,
                                       const void* v_frag, int64_t batch, int32_t seq,
                                       int32_t heads, int32_t kv_heads, int32_t head_dim,
