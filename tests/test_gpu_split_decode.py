@@ -73,6 +73,30 @@ def test_split_decode_attention(monkeypatch, b, H, Hk, d, max_pos, window, posit
     assert ((heads.double() - want).abs() <= 1e-6 * size + 1e-7).all()
 
 
+# the default layers on either side of their line, past the window, and a shape
+# with a line of its own
+@pytest.mark.parametrize("b,H,Hk,d,contexts", [
+    (1, 8, 2, 96, (352, 353, 2500)), (8, 8, 2, 96, (576, 577, 3002)), (2, 8, 8, 96, (768, 769))])
+def test_split_decode_attention_at_its_line(b, H, Hk, d, contexts):
+    """With the rule as it is: the contexts past the line take a workspace, and
+    all agree with the one-launch form as in the tests above."""
+    from parrot import hip_moe
+    max_pos, window, first = 4096, 2048, contexts[1]
+    for context in contexts:
+        print(f"split decode b={b} H={H}/{Hk} context {context}", flush=True)
+        assert (hip_moe.decode_split_bytes(b, H, Hk, d, max_pos, window, context) > 0) == (context >= first)
+        q, kn, vn, kc, vc = _local_inputs(b, H, Hk, d, max_pos, context)
+        pos = torch.tensor([context - 1], dtype=torch.int32, device="cuda")
+        caches = [(kc.clone(), vc.clone()) for _ in range(2)]
+        with torch.no_grad():
+            one, got = (hip_moe.decode_attention(q, kn, vn, *c, pos, window, d ** -0.5, context=known)
+                        for c, known in zip(caches, (None, context)))
+        assert all(torch.equal(x, y) for x, y in zip(*caches))
+        if context < first:
+            assert torch.equal(one, got)
+        assert ((one.double() - got.double()).abs() <= 2 ** -7 * one.double().abs().max()).all()
+
+
 # the NaN key alone in the last chunk, beside others, and in a full first chunk
 @pytest.mark.parametrize("position,nan_key", [(64, 64), (70, 70), (130, 5), (255, 255)])
 def test_split_decode_attention_nan_key(monkeypatch, position, nan_key):
