@@ -69,7 +69,8 @@ __device__ __forceinline__ float hi_bf16(uint32_t w) { return __uint_as_float(w 
 
 // Raw buffer loads: the per-lane byte offset stays fixed over a k loop and
 // the step offset travels in an SGPR, so the loop carries no 64-bit address
-// arithmetic; reads past `bytes` return zero instead of faulting.
+// arithmetic; reads whose per-lane offset lies past `bytes` return zero instead
+// of faulting (the scalar offset alone must stay inside, see extents.h).
 constexpr int kBufferWord3 = 0x00020000;  // gfx9-family buffer resource word 3
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
